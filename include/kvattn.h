@@ -188,13 +188,12 @@ int kva_project_append(kva_cache *cache, int32_t layer, const void *x, int32_t h
                        const void *cos_tab, const void *sin_tab, int32_t table_rows,
                        void *q_out, void *q_gate_out, void *kv_out, kva_stream_t stream);
 /* How the last kva_project_append on this cache projected: steps of up to
- * 64 tokens through the split-K projection kernels and their finish kernel
- * (the weights are read once per 64 tokens); larger steps through one
- * prefill GEMM launch (the reference's batched prefill GEMM,
- * gemm_fp16_prefill.hip:47 at engine.py:3051-3068) whose tiles of 128
- * tokens x one head's 256 weight rows each finish their own rows: fp32 sums
- * rounded to fp16, then the same norm, RoPE and append.  The results
- * satisfy the same contract either way; this says which ran.               */
+ * 64 tokens as split-K products with a finish kernel where that fills the
+ * chip (the weights are read once), larger steps as tiles of one GEMM launch
+ * (the reference's batched prefill GEMM, gemm_fp16_prefill.hip:47 at
+ * engine.py:3051-3068), which finish their own rows unless hidden is split:
+ * fp32 sums rounded to fp16, then the same norm, RoPE and append.  The
+ * results satisfy the same contract either way; this says which ran.       */
 #define KVA_PROJECT_KERNELS 0
 #define KVA_PROJECT_PREFILL_GEMM 1
 int kva_get_project_path(const kva_cache *cache, int32_t *path);

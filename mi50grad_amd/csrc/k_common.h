@@ -132,6 +132,32 @@ __device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t r, uint32_t l
         : "memory", "m0");
 }
 
+// The same with a scalar offset added to every lane's.  A loop that walks k
+// keeps voff in registers for its whole length and moves soff: per-load
+// address arithmetic on the vector unit held a wave's loads to 40-50 GB/s
+// per CU, where this form moves 100-120 (64 KB chunks from L2, 8 waves).
+__device__ __forceinline__ void load_to_lds_at(__amdgpu_buffer_rsrc_t r, uint32_t lds, uint32_t voff, uint32_t soff) {
+    asm volatile(
+        "s_mov_b32 m0, %0\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %1, %2, %3 offen lds"
+        :
+        : "s"(lds), "v"(voff), "s"(r), "s"(soff)
+        : "memory", "m0");
+}
+
+// One dword per lane of a buffer to LDS (lane l's to lds + 4*l), read only to
+// bring its 128-byte line into the XCD's L2.
+__device__ __forceinline__ void touch_line(__amdgpu_buffer_rsrc_t r, uint32_t lds, uint32_t voff, uint32_t soff) {
+    asm volatile(
+        "s_mov_b32 m0, %0\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dword %1, %2, %3 offen lds"
+        :
+        : "s"(lds), "v"(voff), "s"(r), "s"(soff)
+        : "memory", "m0");
+}
+
 // Wait until at most N of this wave's vector-memory operations are
 // outstanding (they complete in order).
 template <int N>
@@ -140,6 +166,13 @@ __device__ __forceinline__ void wait_vm() {
     // s_waitcnt fields: vmcnt[3:0], expcnt[6:4] (7 = no wait), lgkmcnt[11:8]
     // (15 = no wait), vmcnt[5:4] in bits [15:14].
     __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
+}
+
+// The same, and every LDS operation of this wave done.
+template <int N>
+__device__ __forceinline__ void wait_vm_lds() {
+    static_assert(N >= 0 && N < 64, "vmcnt is six bits");
+    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (0 << 8) | ((N >> 4) << 14));
 }
 
 // The XCD (accelerator complex die) this wave runs on: CUs of one XCD

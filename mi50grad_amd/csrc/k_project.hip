@@ -7,23 +7,18 @@
 // (engine.py:2000-2022, 2371-2432; c_dispatch.c:1042-1059 sends V's GEMV
 // straight to the slot).  Here a step's tokens are projected together:
 //
-// proj_gemm_kernel: out[t][n] = sum_k W[n][k] x[t][k] as split-K MFMA tiles.
-//   A workgroup owns a run of 16-row weight tiles and one of `splits`
-//   slices of hidden; each of its waves takes an equal part of the slice for
-//   all those rows and all tokens (up to four 16-token column
-//   tiles), so every weight byte is read from HBM once and x (a few hundred
-//   KB) comes from L2.  The k order inside a 32-wide MFMA step is free as long
-//   as A and B agree: lane group g holds elements 8g..8g+7 of both, 16-byte
-//   loads, 64 contiguous bytes of each weight row per load.  A ring of
-//   register stages with fixed roles keeps several k-steps of loads in
-//   flight ahead of the MFMAs; the last round's extra slots reload cached
-//   weights against zero x instead of branching, so the compiler's
-//   load-counter waits never drain the loads in flight.  The waves' sums
-//   meet in LDS in a fixed order and go out as fp32 partials
-//   [split][token][row].  proj_lds_kernel, the form for up to 32 tokens,
-//   keeps x in registers and stages the weights through LDS instead.
-// proj_finish_kernel: per (token, head), one 32-lane group sums the splits
-//   in order, rounds to fp16 and then does what the append kernel does:
+// out[t][n] = sum_k W[n][k] x[t][k], in one of two forms (launch_product):
+// - proj_lds_kernel, up to 32 tokens of the hidden sizes it is built for: a
+//   workgroup owns a run of 16-row weight tiles and one of `splits` slices of
+//   hidden, each of its waves an equal part of the slice for all those rows
+//   and all tokens, x in registers and the weights streamed through LDS, so
+//   every weight byte is read from HBM once.  The k order inside a 32-wide
+//   MFMA step is free as long as A and B agree: lane group g holds elements
+//   8g..8g+7 of both.  The waves' sums meet in LDS in a fixed order and go
+//   out as fp32 partials [split][token][row].
+// - the LDS-tiled GEMMs of k_gemm.hip for everything else.
+// proj_finish_kernel, where hidden was split: per (token, head), one
+//   32-lane group sums the splits in order, rounds to fp16 and then does what the append kernel does:
 //   Q -> norm + RoPE -> q_out, Q_gate -> gate_out, K -> norm + RoPE -> its
 //   page slot, V -> its page slot (and K, V as projected -> kv_out).
 #include "k_common.h"
@@ -34,33 +29,6 @@ namespace kva {
 namespace {
 
 __device__ __forceinline__ half8_t as_h8(uint4 v) { return __builtin_bit_cast(half8_t, v); }
-
-template <int NTB, int RT>
-struct ProjStage {
-    uint4 w[RT];   // 16-row weight tiles: row 16*i + lane%16, 8 elements
-    uint4 x[NTB];  // 16-token tiles: token 16*j + lane%16, the same 8 elements
-};
-
-// This workgroup's weight row tiles: tile i holds rows 16*(grp*RT + i) ..
-// +15 of the stacked [w_a; w_b] (a tile never straddles the two: n_a is a
-// multiple of 16).  Tiles past the last one repeat it (live = false: loaded,
-// never written), so every wave issues the same loads.  wt[i] points at
-// this lane's row and first element.
-template <int RT>
-__device__ __forceinline__ void proj_tiles(const ProjectArgs &a, int grp, int lane_off,
-                                           const uint16_t *(&wt)[RT], bool (&live)[RT]) {
-    const int n_t16 = (a.n_a + a.n_b) / 16;
-    const size_t hidden = static_cast<size_t>(a.hidden);
-#pragma unroll
-    for (int i = 0; i < RT; ++i) {
-        const int t16 = grp * RT + i;
-        live[i] = t16 < n_t16;
-        const int row = 16 * min(t16, n_t16 - 1);
-        const uint16_t *base = row < a.n_a ? a.w_a + static_cast<size_t>(row) * hidden
-                                           : a.w_b + static_cast<size_t>(row - a.n_a) * hidden;
-        wt[i] = base + lane_off;
-    }
-}
 
 // Sum the waves' k ranges, one row tile at a time through LDS, in wave
 // order; wave i % WAVES writes row tile i's partial [split][token][row].
@@ -91,90 +59,6 @@ __device__ __forceinline__ void proj_reduce_store(const ProjectArgs &a, float4_t
         }
         __syncthreads();
     }
-}
-
-// Load k-step `step` of this wave into a stage.  Steps past the wave's
-// range (the ring's last round) reload the final step's weights (cache hits)
-// and read x out of range (zeros), so their MFMAs add nothing and every
-// round issues the same loads: no branch, exact load-counter waits.
-template <int NTB, int RT>
-__device__ __forceinline__ void proj_load(ProjStage<NTB, RT> &st, const uint16_t *const (&wt)[RT],
-                                          __amdgpu_buffer_rsrc_t xr, const uint32_t (&xoff)[NTB], int step,
-                                          int steps) {
-    const int ks = min(step, steps - 1);
-#pragma unroll
-    for (int i = 0; i < RT; ++i) st.w[i] = ld16(wt[i] + 32 * ks);
-#pragma unroll
-    for (int j = 0; j < NTB; ++j) {
-        const uint32_t off = step < steps ? xoff[j] + 64u * static_cast<uint32_t>(ks) : 0x80000000u;
-        const auto v = __builtin_amdgcn_raw_buffer_load_b128(xr, off, 0, 0);
-        st.x[j] = make_uint4(v[0], v[1], v[2], v[3]);
-    }
-}
-
-template <int NTB, int RT>
-__device__ __forceinline__ void proj_mfma(float4_t (&acc)[RT][NTB], const ProjStage<NTB, RT> &st) {
-#pragma unroll
-    for (int i = 0; i < RT; ++i)
-#pragma unroll
-        for (int j = 0; j < NTB; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(st.w[i]), as_h8(st.x[j]), acc[i][j], 0, 0, 0);
-}
-
-// General form.  Grid: ceil(rows / (16 * RT)) * splits workgroups of WAVES
-// waves; each wave covers all 16 * RT rows of its workgroup for
-// hidden / (splits * WAVES) elements of k.  The host checks
-// hidden % (32 * WAVES * splits) == 0 and n_tok <= 16 * NTB.  A ring of
-// DEPTH + 1 stages keeps DEPTH k-steps of loads in flight while one is
-// multiplied.
-template <int NTB, int WAVES, int DEPTH, int RT>
-__global__ __launch_bounds__(64 * WAVES) void proj_gemm_kernel(ProjectArgs a) {
-    constexpr int R = DEPTH + 1;
-    __shared__ float4_t red[WAVES][NTB][64];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int n_grp = ((a.n_a + a.n_b) / 16 + RT - 1) / RT;
-    const int grp = blockIdx.x % n_grp;
-    const int split = blockIdx.x / n_grp;
-    const int steps = a.hidden / (32 * WAVES * a.splits);  // k-steps of this wave
-    const int k0 = (split * WAVES + wave) * steps * 32;
-    const int r = lane & 15, g = lane >> 4;
-    const uint16_t *wt[RT];
-    bool live[RT];
-    proj_tiles<RT>(a, grp, r * a.hidden + k0 + 8 * g, wt, live);
-    // x rows past n_tok lie outside the resource and load as zeros.
-    const auto xr = ro_rsrc(a.x, static_cast<uint32_t>(a.n_tok) * static_cast<uint32_t>(a.hidden) * 2u);
-    uint32_t xoff[NTB];
-#pragma unroll
-    for (int j = 0; j < NTB; ++j) xoff[j] = ((16 * j + r) * static_cast<uint32_t>(a.hidden) + k0 + 8 * g) * 2u;
-
-    float4_t acc[RT][NTB];
-#pragma unroll
-    for (int i = 0; i < RT; ++i)
-#pragma unroll
-        for (int j = 0; j < NTB; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
-
-    // Slot j of round rr holds step rr*R + j.  Scheduling barriers keep each
-    // group of loads ahead of the MFMAs after it; left alone, the scheduler
-    // interleaves them and only a few loads stay in flight.
-    ProjStage<NTB, RT> st[R];
-#pragma unroll
-    for (int j = 0; j < DEPTH; ++j) {
-        __builtin_amdgcn_sched_barrier(0);
-        proj_load(st[j], wt, xr, xoff, j, steps);
-    }
-    const int rounds = (steps + R - 1) / R;
-    for (int rr = 0; rr < rounds; ++rr) {
-#pragma unroll
-        for (int j = 0; j < R; ++j) {
-            __builtin_amdgcn_sched_barrier(0);
-            proj_load(st[(j + DEPTH) % R], wt, xr, xoff, rr * R + j + DEPTH, steps);
-            __builtin_amdgcn_sched_barrier(0);
-            proj_mfma(acc, st[j]);
-        }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    proj_reduce_store<NTB, WAVES, RT>(a, acc, red, live, grp, split, wave, lane);
 }
 
 // The form for up to 32 tokens and STEPS k-steps per wave: each wave's x
@@ -298,15 +182,15 @@ __global__ __launch_bounds__(64 * WAVES) void proj_lds_kernel(ProjectArgs a) {
 // value heads (the order of the weight rows).  The token's metadata and
 // page id are workgroup-uniform, read through the scalar cache while the
 // partials are in flight.
+template <int S>
 __global__ __launch_bounds__(256) void proj_finish_kernel(ProjectArgs a) {
     const int H = a.num_heads, hkv = a.num_kv_heads;
     const int rows_per_tok = 2 * H + 2 * hkv;
     const int blocks_per_tok = (rows_per_tok + 7) / 8;
-    const int tc = blockIdx.x / blocks_per_tok;
-    const int hr = (blockIdx.x - tc * blocks_per_tok) * 8 + (threadIdx.x >> 5);
+    const int t = blockIdx.x / blocks_per_tok;
+    const int hr = (blockIdx.x - t * blocks_per_tok) * 8 + (threadIdx.x >> 5);
     const int lane = threadIdx.x & 31;
     if (hr >= rows_per_tok) return;  // whole 32-lane group leaves
-    const int t = a.tok0 + tc;
     // Two memory round trips before the stores.  First: every split's
     // partial (splits past a.splits reread split 0 and are not added) and
     // the norm weights, which need only the kernel arguments, with the
@@ -314,12 +198,12 @@ __global__ __launch_bounds__(256) void proj_finish_kernel(ProjectArgs a) {
     // (Requested in source order, the partials waited for the page id, which
     // waited for the sequence and slot: three round trips.)
     const size_t N = static_cast<size_t>(a.n_a) + a.n_b;
-    const size_t row_at = static_cast<size_t>(tc) * N + static_cast<size_t>(hr) * kHeadDim + 8 * lane;
+    const size_t row_at = static_cast<size_t>(t) * N + static_cast<size_t>(hr) * kHeadDim + 8 * lane;
     const size_t split_stride = static_cast<size_t>(a.n_tok) * N;
     const int splits = a.splits;
-    float4_t plo[kProjMaxSplits], phi[kProjMaxSplits];
+    float4_t plo[S], phi[S];
 #pragma unroll
-    for (int s = 0; s < kProjMaxSplits; ++s) {
+    for (int s = 0; s < S; ++s) {
         const float *ps = a.part + row_at + (s < splits ? s : 0) * split_stride;
         plo[s] = *reinterpret_cast<const float4_t *>(ps);
         phi[s] = *reinterpret_cast<const float4_t *>(ps + 4);
@@ -340,7 +224,7 @@ __global__ __launch_bounds__(256) void proj_finish_kernel(ProjectArgs a) {
     {
         float4_t lo = plo[0], hi = phi[0];
 #pragma unroll
-        for (int s = 1; s < kProjMaxSplits; ++s) {
+        for (int s = 1; s < S; ++s) {
             lo = s < splits ? lo + plo[s] : lo;
             hi = s < splits ? hi + phi[s] : hi;
         }
@@ -375,27 +259,28 @@ __global__ __launch_bounds__(256) void proj_finish_kernel(ProjectArgs a) {
 // residual add, the epilogue of the reference GEMV (gemv_fp16_v2.hip:81-86).
 // A thread reads its residual before writing the same 16 bytes, so the
 // residual may be the output (in place, d_hidden += o_proj(attn)).
+template <int S>
 __global__ __launch_bounds__(256) void oproj_finish_kernel(ProjectArgs a) {
     const int per_tok = a.n_a / 8;
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= a.n_tok * per_tok) return;
-    const int tc = i / per_tok;
+    const int t = i / per_tok;
     const size_t N = static_cast<size_t>(a.n_a);
-    const size_t row = static_cast<size_t>(i - tc * per_tok) * 8;
-    const size_t at = static_cast<size_t>(a.tok0 + tc) * N + row;
+    const size_t row = static_cast<size_t>(i - t * per_tok) * 8;
+    const size_t at = static_cast<size_t>(t) * N + row;
     const uint4 r = a.residual ? ld16(a.residual + at) : make_uint4(0, 0, 0, 0);
     const size_t split_stride = static_cast<size_t>(a.n_tok) * N;
-    const float *p = a.part + static_cast<size_t>(tc) * N + row;
-    float4_t plo[kProjMaxSplits], phi[kProjMaxSplits];
+    const float *p = a.part + at;
+    float4_t plo[S], phi[S];
 #pragma unroll
-    for (int s = 0; s < kProjMaxSplits; ++s) {
+    for (int s = 0; s < S; ++s) {
         const float *ps = p + (s < a.splits ? s : 0) * split_stride;
         plo[s] = *reinterpret_cast<const float4_t *>(ps);
         phi[s] = *reinterpret_cast<const float4_t *>(ps + 4);
     }
     float4_t lo = plo[0], hi = phi[0];
 #pragma unroll
-    for (int s = 1; s < kProjMaxSplits; ++s) {
+    for (int s = 1; s < S; ++s) {
         lo = s < a.splits ? lo + plo[s] : lo;
         hi = s < a.splits ? hi + phi[s] : hi;
     }
@@ -411,61 +296,77 @@ __global__ __launch_bounds__(256) void oproj_finish_kernel(ProjectArgs a) {
     st16(a.y_out + at, y);
 }
 
+// Whether the x-resident form serves this call: few enough tokens for x to
+// stay in registers, and a hidden size that gives every wave one of the two
+// built step counts.  It streams the weights at 5.1 TB/s where a GEMM tile of
+// 64 tokens reaches 4.5 (one token, hidden 5120, 14336 rows: 28.7 us against
+// 28.9 to 33.8); past 32 tokens x no longer fits beside the sums.
+bool streams(const ProjectArgs &a) {
+    const int per_step = 32 * kProjWaves * a.splits;
+    return a.n_tok <= kProjStreamTokens &&
+           (a.hidden == kProjStreamSteps * per_step || a.hidden == kProjStreamStepsB * per_step);
+}
+
 // Split-K partials of x [n_tok][hidden] against the stacked weight rows.
-hipError_t launch_proj_gemm(const ProjectArgs &a, hipStream_t s) {
-    constexpr int W = kProjWaves, P = kProjDepth, RT = kProjRowTiles, LD = kProjLdsDepth;
-    const int n_t16 = (a.n_a + a.n_b) / 16;
-    const dim3 grid(static_cast<unsigned>((n_t16 + RT - 1) / RT * a.splits));
-    const dim3 block(64 * W);
-    const int ntb = (a.n_tok + 15) / 16;
-    if (ntb <= 2 && a.hidden == kProjStreamSteps * 32 * W * a.splits) {
-        constexpr int ST = kProjStreamSteps;
-        if (ntb == 1) hipLaunchKernelGGL((proj_lds_kernel<1, W, RT, ST, LD>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((proj_lds_kernel<2, W, RT, ST, LD>), grid, block, 0, s, a);
-    } else if (ntb <= 2 && a.hidden == kProjStreamStepsB * 32 * W * a.splits) {
-        constexpr int ST = kProjStreamStepsB, RB = kProjRowTilesB;
-        const dim3 grid_b(static_cast<unsigned>((n_t16 + RB - 1) / RB * a.splits));
-        if (ntb == 1) hipLaunchKernelGGL((proj_lds_kernel<1, W, RB, ST, LD>), grid_b, block, 0, s, a);
-        else hipLaunchKernelGGL((proj_lds_kernel<2, W, RB, ST, LD>), grid_b, block, 0, s, a);
-    } else switch (ntb) {
-        case 1: hipLaunchKernelGGL((proj_gemm_kernel<1, W, P, RT>), grid, block, 0, s, a); break;
-        case 2: hipLaunchKernelGGL((proj_gemm_kernel<2, W, P, RT>), grid, block, 0, s, a); break;
-        case 3: hipLaunchKernelGGL((proj_gemm_kernel<3, W, P, RT>), grid, block, 0, s, a); break;
-        case 4: hipLaunchKernelGGL((proj_gemm_kernel<4, W, P, RT>), grid, block, 0, s, a); break;
-        default: return hipErrorInvalidValue;
-    }
+hipError_t launch_stream(const ProjectArgs &a, hipStream_t s) {
+    constexpr int W = kProjWaves, LD = kProjLdsDepth;
+    constexpr int SA = kProjStreamSteps, RA = kProjRowTiles, SB = kProjStreamStepsB, RB = kProjRowTilesB;
+    const bool form_a = a.hidden == SA * 32 * W * a.splits;
+    const int n_t16 = (a.n_a + a.n_b) / 16, rt = form_a ? RA : RB;
+    const dim3 grid(static_cast<unsigned>((n_t16 + rt - 1) / rt * a.splits)), block(64 * W);
+    const bool one = a.n_tok <= 16;
+    if (form_a && one) hipLaunchKernelGGL((proj_lds_kernel<1, W, RA, SA, LD>), grid, block, 0, s, a);
+    else if (form_a) hipLaunchKernelGGL((proj_lds_kernel<2, W, RA, SA, LD>), grid, block, 0, s, a);
+    else if (one) hipLaunchKernelGGL((proj_lds_kernel<1, W, RB, SB, LD>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((proj_lds_kernel<2, W, RB, SB, LD>), grid, block, 0, s, a);
     return hipGetLastError();
 }
 
-}  // namespace
-
-// The GEMM of a launch pair between the caller's timing events (if any).
-hipError_t launch_proj_gemm_timed(const ProjectArgs &a, hipStream_t s) {
+// The product, between the caller's timing events (if any); `partial` is set
+// when it leaves partials for a finish kernel.
+hipError_t launch_product(ProjectArgs &a, bool heads, int n_cu, size_t part_floats, bool &partial, hipStream_t s) {
     if (a.ev_before) {
         const hipError_t e = hipEventRecord(a.ev_before, s);
         if (e != hipSuccess) return e;
     }
-    const hipError_t e = launch_proj_gemm(a, s);
+    hipError_t e;
+    if (streams(a)) {
+        partial = true;
+        e = launch_stream(a, s);
+    } else {
+        e = launch_gemm_project(a, heads, n_cu, part_floats, s);
+        partial = a.splits > 1;
+    }
     if (e != hipSuccess || !a.ev_after) return e;
     return hipEventRecord(a.ev_after, s);
 }
 
-hipError_t launch_project(const ProjectArgs &a, hipStream_t s) {
+}  // namespace
+
+hipError_t launch_project(ProjectArgs a, int n_cu, size_t part_floats, hipStream_t s) {
     if (a.n_tok <= 0) return hipSuccess;
-    const hipError_t e = launch_proj_gemm_timed(a, s);
-    if (e != hipSuccess) return e;
+    bool partial = false;
+    const hipError_t e = launch_product(a, true, n_cu, part_floats, partial, s);
+    if (e != hipSuccess || !partial) return e;
     const int blocks_per_tok = (2 * a.num_heads + 2 * a.num_kv_heads + 7) / 8;
-    hipLaunchKernelGGL(proj_finish_kernel, dim3(a.n_tok * blocks_per_tok), dim3(256), 0, s, a);
+    const dim3 grid(static_cast<unsigned>(a.n_tok) * blocks_per_tok), block(256);
+    if (a.splits <= 2) hipLaunchKernelGGL(proj_finish_kernel<2>, grid, block, 0, s, a);
+    else if (a.splits <= 4) hipLaunchKernelGGL(proj_finish_kernel<4>, grid, block, 0, s, a);
+    else hipLaunchKernelGGL(proj_finish_kernel<kGemmMaxSplits>, grid, block, 0, s, a);
     return hipGetLastError();
 }
 
-hipError_t launch_out_project(const ProjectArgs &a, hipStream_t s) {
+hipError_t launch_out_project(ProjectArgs a, int n_cu, size_t part_floats, hipStream_t s) {
     if (a.n_tok <= 0) return hipSuccess;
     if (a.n_b != 0 || a.n_a % 16 != 0) return hipErrorInvalidValue;
-    const hipError_t e = launch_proj_gemm_timed(a, s);
-    if (e != hipSuccess) return e;
-    const int threads = a.n_tok * (a.n_a / 8);
-    hipLaunchKernelGGL(oproj_finish_kernel, dim3((threads + 255) / 256), dim3(256), 0, s, a);
+    bool partial = false;
+    const hipError_t e = launch_product(a, false, n_cu, part_floats, partial, s);
+    if (e != hipSuccess || !partial) return e;
+    const int64_t threads = static_cast<int64_t>(a.n_tok) * (a.n_a / 8);
+    const dim3 grid(static_cast<unsigned>((threads + 255) / 256)), block(256);
+    if (a.splits <= 2) hipLaunchKernelGGL(oproj_finish_kernel<2>, grid, block, 0, s, a);
+    else if (a.splits <= 4) hipLaunchKernelGGL(oproj_finish_kernel<4>, grid, block, 0, s, a);
+    else hipLaunchKernelGGL(oproj_finish_kernel<kGemmMaxSplits>, grid, block, 0, s, a);
     return hipGetLastError();
 }
 

@@ -83,8 +83,9 @@ struct kva_cache {
     float *d_mq_acc = nullptr;  // multi-query partial slots [2*mq_max_wg][8][16][256]
     float *d_mq_ml = nullptr;
     int32_t mq_max_wg = 0;
-    float *d_proj = nullptr;    // projection partials [kProjMaxSplits][kProjTokens][(2H+2Hkv)*256]
-    size_t proj_floats = 0;
+    float *d_proj = nullptr;    // projection partials [splits][tokens][rows]
+    size_t part_floats = 0;     // what it holds
+    size_t proj_floats = 0;     // the partials that kva_out_project's refusals are counted in
     int32_t last_proj_path = 0;  // KVA_PROJECT_KERNELS or KVA_PROJECT_PREFILL_GEMM
     int32_t max_wg = 0;  // decode workgroups the partial workspace can serve
     size_t ws_rows = 0;  // 256-float rows in the decode partial workspace
@@ -368,6 +369,7 @@ int kva_create(const kva_config *cfg, kva_cache **out) {
     // device (against a nominal MI355X CU count) before they are refused.
     c->proj_floats = static_cast<size_t>(kva::kProjMaxSplits) * kva::kProjTokens *
                      (2 * static_cast<size_t>(cfg->num_heads) + 2 * cfg->num_kv_heads) * kva::kHeadDim;
+    c->part_floats = kva::kProjPartFactor * c->proj_floats;
     c->n_cu = kHostOnlyCus;
     c->mq_max_wg = c->n_cu;  // the device's CU count below
     if (!c->host_only) {
@@ -408,7 +410,7 @@ int kva_create(const kva_config *cfg, kva_cache **out) {
             return cleanup(hip_fail(e, "hipMalloc(multi-query workspace)"));
         if ((e = hipMalloc(&c->d_mq_ml, mq_rows * 2 * sizeof(float))) != hipSuccess)
             return cleanup(hip_fail(e, "hipMalloc(multi-query workspace ml)"));
-        if ((e = hipMalloc(&c->d_proj, c->proj_floats * sizeof(float))) != hipSuccess)
+        if ((e = hipMalloc(&c->d_proj, c->part_floats * sizeof(float))) != hipSuccess)
             return cleanup(hip_fail(e, "hipMalloc(projection workspace)"));
         for (int i = 0; i < kStageSlots; ++i) {
             if ((e = hipHostMalloc(reinterpret_cast<void **>(&c->h_stage[i]), c->stage_bytes,
@@ -963,27 +965,10 @@ static int project_impl(kva_cache *c, int32_t layer, const void *x, int32_t hidd
     a.eps = c->cfg.eps;
     a.ev_before = c->kev_before;
     a.ev_after = c->kev_after;
-    const auto *xs = static_cast<const uint16_t *>(x);
-    const hipStream_t s = static_cast<hipStream_t>(stream);
-    // Prefill-sized steps: one GEMM launch whose tiles are whole heads, the
-    // epilogue fused (the reference's batched path at seq_len >= 32,
-    // engine.py:3051-3068), instead of 64-token launch pairs that would
-    // each read all the weights.
-    if (c->st_n_tok > kva::kProjTokens) {
-        a.tok0 = 0;
-        a.n_tok = c->st_n_tok;
-        a.x = xs;
-        KVA_HIP(kva::launch_project_big(a, s));
-        c->last_proj_path = KVA_PROJECT_PREFILL_GEMM;
-        return KVA_OK;
-    }
-    for (int32_t t0 = 0; t0 < c->st_n_tok; t0 += kva::kProjTokens) {
-        a.tok0 = t0;
-        a.n_tok = std::min(kva::kProjTokens, c->st_n_tok - t0);
-        a.x = xs + static_cast<size_t>(t0) * hidden;
-        KVA_HIP(kva::launch_project(a, s));
-    }
-    c->last_proj_path = KVA_PROJECT_KERNELS;
+    a.x = static_cast<const uint16_t *>(x);
+    a.n_tok = c->st_n_tok;
+    KVA_HIP(kva::launch_project(a, c->n_cu, c->part_floats, static_cast<hipStream_t>(stream)));
+    c->last_proj_path = c->st_n_tok > kva::kProjTokens ? KVA_PROJECT_PREFILL_GEMM : KVA_PROJECT_KERNELS;
     return KVA_OK;
 }
 
@@ -1310,13 +1295,9 @@ static int out_project_impl(kva_cache *c, const void *attn, int32_t n_tok, int32
     a.ev_after = c->kev_after;
     a.y_out = static_cast<uint16_t *>(out);
     a.residual = static_cast<const uint16_t *>(residual);
-    const auto *xs = static_cast<const uint16_t *>(attn);
-    for (int32_t t0 = 0; t0 < n_tok; t0 += kva::kProjTokens) {
-        a.tok0 = t0;
-        a.n_tok = std::min(kva::kProjTokens, n_tok - t0);
-        a.x = xs + static_cast<size_t>(t0) * q_dim;
-        KVA_HIP(kva::launch_out_project(a, static_cast<hipStream_t>(stream)));
-    }
+    a.x = static_cast<const uint16_t *>(attn);
+    a.n_tok = n_tok;
+    KVA_HIP(kva::launch_out_project(a, c->n_cu, c->part_floats, static_cast<hipStream_t>(stream)));
     return KVA_OK;
 }
 

@@ -45,18 +45,23 @@ hipError_t launch_append(const AppendArgs &a, hipStream_t s);
 
 // Q/K/V projection of a step's tokens fused with norm + RoPE + K/V append.
 // Weight rows: w_a = [Q heads | Q_gate heads] (n_a = 2*H*256 rows), w_b =
-// [K heads | V heads] (n_b = 2*Hkv*256 rows), each row `hidden` fp16.  One
-// launch pair covers up to kProjTokens tokens: proj_gemm_kernel writes
-// split-K fp32 partials, proj_finish_kernel sums them in split order, rounds
-// to fp16 (the projection the reference's GEMV stores) and finishes each head.
-constexpr int kProjTokens = 64;     // tokens per launch pair (4 MFMA column tiles)
-constexpr int kProjMaxSplits = 4;   // hidden split among workgroups, at most
-constexpr int kProjWaves = 8;       // waves per GEMM workgroup
-constexpr int kProjRowTiles = 7;    // 16-row weight tiles per GEMM workgroup
-constexpr int kProjDepth = 1;       // k-steps of loads in flight per wave (general form)
+// [K heads | V heads] (n_b = 2*Hkv*256 rows), each row `hidden` fp16.  Up to
+// 32 tokens of the hidden sizes that fit it stream the weights past x held
+// in registers (proj_lds_kernel); everything else runs as LDS-tiled GEMMs
+// (k_gemm.hip).  A form that splits hidden among workgroups writes fp32
+// partials, and a finish kernel sums them in split order, rounds to fp16
+// (the projection the reference's GEMV stores) and finishes each head; an
+// unsplit GEMM does that in its own epilogue.
+constexpr int kProjTokens = 64;     // tokens the workspace refusals are counted in
+constexpr int kProjMaxSplits = 4;   // hidden split among workgroups, at most (proj_lds_kernel)
+constexpr int kGemmMaxSplits = 8;   // the same of the GEMM forms
+constexpr int kProjPartFactor = 4;  // partial workspace over kProjMaxSplits x kProjTokens tokens of every row
+constexpr int kProjWaves = 8;       // waves per workgroup
+constexpr int kProjRowTiles = 7;    // 16-row weight tiles per workgroup
 constexpr int kProjHiddenQuantum = 512;  // hidden must be a multiple of this
-constexpr int kProjWgPerCu = 1;     // GEMM workgroups per CU the split aims for, at most
-constexpr int kProjStreamSteps = 10;  // k-steps per wave of the x-resident form (up to 32 tokens)
+constexpr int kProjWgPerCu = 1;     // workgroups per CU the split aims for, at most
+constexpr int kProjStreamTokens = 32; // most tokens of the x-resident form
+constexpr int kProjStreamSteps = 10;  // its k-steps per wave
 constexpr int kProjLdsDepth = 6;      // two-step LDS stages in flight per wave there
 // The same form over 6 k-steps per wave (hidden 6144 at four splits: the
 // O-projection from 24 heads), with 5 row tiles per workgroup so that 5120
@@ -64,15 +69,14 @@ constexpr int kProjLdsDepth = 6;      // two-step LDS stages in flight per wave 
 constexpr int kProjStreamStepsB = 6;
 constexpr int kProjRowTilesB = 5;
 struct ProjectArgs {
-    const uint16_t *x;        // [n_tok][hidden], this chunk's first token
+    const uint16_t *x;        // [n_tok][hidden]
     const uint16_t *w_a;
     const uint16_t *w_b;
     int32_t n_a, n_b;
     int32_t hidden;
-    int32_t n_tok;            // tokens of this chunk, 1..kProjTokens
-    int32_t splits;
+    int32_t n_tok;
+    int32_t splits;           // of hidden among workgroups
     float *part;              // [splits][n_tok][n_a + n_b]
-    int32_t tok0;             // the chunk's first token within the step
     uint16_t *q_out;          // [T][H][256]: normalised + rotated Q
     uint16_t *gate_out;       // [T][H][256]: Q_gate as projected (nullable)
     uint16_t *kv_out;         // [T][2][Hkv][256]: K, V as projected (nullable)
@@ -99,16 +103,15 @@ struct ProjectArgs {
     // DecodeArgs.
     hipEvent_t ev_before, ev_after;
 };
-hipError_t launch_project(const ProjectArgs &a, hipStream_t s);
-hipError_t launch_out_project(const ProjectArgs &a, hipStream_t s);
-// Prefill-sized steps (more than kProjTokens tokens): one GEMM launch over
-// every token, tiles of kBigTileTokens tokens x one head's 256 weight rows,
-// with the finish kernel's epilogue (fp16 rounding, norm + RoPE, outputs,
-// cache rows) done by the workgroup that computed the tile (k_gemm.hip).
-// Needs (n_a + n_b) % 256 == 0 and hidden % 64 == 0; a.tok0 = 0.
-constexpr int kBigTileTokens = 256;
+// `a.splits` is the split of the x-resident form; part_floats what a.part
+// holds (the GEMM forms choose their own split from it and the CU count).
+hipError_t launch_project(ProjectArgs a, int n_cu, size_t part_floats, hipStream_t s);
+hipError_t launch_out_project(ProjectArgs a, int n_cu, size_t part_floats, hipStream_t s);
+// The LDS-tiled GEMM of either (k_gemm.hip): heads, the Q/K/V projection;
+// else the O-projection.  Sets a.splits: 1, the outputs are written; more,
+// a.part holds that many partials.  Needs hidden % 64 == 0.
 constexpr int kBigProjMaxTokens = 1 << 24;
-hipError_t launch_project_big(const ProjectArgs &a, hipStream_t s);
+hipError_t launch_gemm_project(ProjectArgs &a, bool heads, int n_cu, size_t part_floats, hipStream_t s);
 
 // Reference-compatible norm+RoPE on a contiguous [n_heads][head_dim] buffer.
 struct LegacyNormArgs {

@@ -1,0 +1,53 @@
+"""GPU: the tile GEMMs behind kva_out_project and kva_project_append at the
+edges of their tiles (64, 128 and 256 tokens; 128, 256 and 320 rows), with
+and without a split of hidden, on inputs whose fp32 sums are exact, so every
+output is bit-exact whatever the tile, split or order."""
+import numpy as np
+import pytest
+
+from oracle import kvattn_oracle as orc
+
+from gpu_helpers import Tables, build_cache, say
+from test_gpu_oproj import _inputs
+from test_gpu_project import _check_cache_rows, _run
+
+pytestmark = pytest.mark.gpu
+
+
+def _bits(a):
+    return a.view(np.uint16)
+
+
+# Rows past the last tile (16, 80 and 336 of 128, 256 or 320), token
+# remainders of 1, 8 and 44, one round and several, one split and several.
+@pytest.mark.parametrize("n_tok,q_dim,n_out", [(33, 512, 16), (64, 6144, 336), (65, 1536, 5120), (129, 6144, 80),
+                                               (200, 6144, 5120), (700, 6144, 5120), (1300, 512, 5120)])
+def test_out_project_tiles_exact(device, n_tok, q_dim, n_out):
+    rng = np.random.default_rng(n_tok + n_out)
+    say(f"out_project tiles n_tok={n_tok} q_dim={q_dim} n_out={n_out}")
+    cache, _, _ = build_cache([8], [[0]], extra_rows=[1])
+    x, w, r = _inputs(rng, n_tok, q_dim, n_out, True)
+    guard = np.full((1, n_out), 77.0, np.float16)  # a row past the output stays as it was
+    out = device.array(np.concatenate([r, guard]))
+    cache.out_project(device.array(x), n_tok, q_dim, device.array(w), n_out, out, residual=out)
+    device.synchronize()
+    got = out.numpy()
+    assert np.array_equal(_bits(got[:n_tok]), _bits(orc.out_project(x, w, r)))
+    assert np.array_equal(_bits(got[n_tok:]), _bits(guard))
+    cache.destroy()
+
+
+@pytest.mark.parametrize("hidden,n_new", [(512, [33]), (5120, [64]), (5120, [50, 79]), (2560, [300])])
+def test_project_tiles_exact(device, hidden, n_new):
+    rng = np.random.default_rng(hidden + sum(n_new))
+    lengths = [int(x) for x in rng.integers(0, 60, len(n_new))]
+    say(f"project_append tiles hidden {hidden}, n_new {n_new}")
+    tables = Tables(device, 512)
+    cache, kr, vr, exp, got, _, _, _, _ = _run(device, rng, lengths, n_new, hidden, True, tables)
+    q, gate, k_raw, k, v = exp
+    assert np.array_equal(_bits(got["kv"][:, 0]), _bits(k_raw))
+    assert np.array_equal(_bits(got["kv"][:, 1]), _bits(v))
+    assert np.array_equal(_bits(got["g"]), _bits(gate))
+    assert np.array_equal(_bits(got["q"]), _bits(q))
+    _check_cache_rows(cache, kr, vr, lengths, n_new, k, v)
+    cache.destroy()
