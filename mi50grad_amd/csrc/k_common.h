@@ -219,28 +219,6 @@ __device__ __forceinline__ float group4_sum(float x) {
     return a + b;
 }
 
-// Four attention output dims o0..o3 as fp16, through the optional output
-// gate: the attention value is rounded to fp16 first and then multiplied by
-// 1/(1+exp(-g)) in float32 (sigmoid_mul.hip:10-22 applied to the attention
-// output, engine.py:2055-2056 after decode and :3120-3121 after prefill), so
-// the fused result equals the reference's two launches.  g4: the four gate
-// values (8-byte aligned) or null.
-__device__ __forceinline__ uint2 out_fp16x4(float o0, float o1, float o2, float o3, const uint16_t *g4) {
-    uint2 o;
-    o.x = pack_h2(o0, o1);
-    o.y = pack_h2(o2, o3);
-    if (!g4) return o;
-    const uint2 gw = *reinterpret_cast<const uint2 *>(g4);
-    const float g[4] = {lo_f(gw.x), hi_f(gw.x), lo_f(gw.y), hi_f(gw.y)};
-    const float a[4] = {lo_f(o.x), hi_f(o.x), lo_f(o.y), hi_f(o.y)};
-    float r[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) r[i] = a[i] * (1.0f / (1.0f + expf(-g[i])));
-    o.x = pack_h2(r[0], r[1]);
-    o.y = pack_h2(r[2], r[3]);
-    return o;
-}
-
 __device__ __forceinline__ uint4 ld16(const uint16_t *p) {
     return *reinterpret_cast<const uint4 *>(p);
 }
@@ -249,6 +227,36 @@ __device__ __forceinline__ uint2 ld8(const uint16_t *p) {
 }
 __device__ __forceinline__ void st16(uint16_t *p, uint4 v) {
     *reinterpret_cast<uint4 *>(p) = v;
+}
+
+// Four attention output dims o0..o3 as fp16.
+__device__ __forceinline__ uint2 pack_out4(float o0, float o1, float o2, float o3) {
+    return make_uint2(pack_h2(o0, o1), pack_h2(o2, o3));
+}
+
+// The output gate on four fp16 attention outputs: each is multiplied by
+// 1/(1+exp(-g)) in float32 and rounded once more (sigmoid_mul.hip:10-22
+// applied to the attention output, engine.py:2055-2056 after decode and
+// :3120-3121 after prefill), so the fused result equals the reference's two
+// launches.  exp and the reciprocal are the hardware's (v_exp_f32,
+// v_rcp_f32, 1 ulp each): the float32 error, about 1e-6, stays far below the
+// fp16 rounding.  expf and an IEEE division are some 40 instructions per
+// value and made the gate 43 of the 174 us of a prefill of 4 x 512 tokens.
+__device__ __forceinline__ uint2 gate4(uint2 o, uint2 gw) {
+    const float g[4] = {lo_f(gw.x), hi_f(gw.x), lo_f(gw.y), hi_f(gw.y)};
+    const float a[4] = {lo_f(o.x), hi_f(o.x), lo_f(o.y), hi_f(o.y)};
+    float r[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        r[i] = a[i] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g[i] * -1.4426950408889634f));
+    return pack_out4(r[0], r[1], r[2], r[3]);
+}
+
+// Four attention output dims as fp16, through the gate at g4 (8-byte
+// aligned) unless it is null.
+__device__ __forceinline__ uint2 out_fp16x4(float o0, float o1, float o2, float o3, const uint16_t *g4) {
+    const uint2 o = pack_out4(o0, o1, o2, o3);
+    return g4 ? gate4(o, ld8(g4)) : o;
 }
 
 }  // namespace kva

@@ -20,8 +20,9 @@
 //   whole tiles would leave most of the 256 CUs idle.
 // The O-projection of 2048 tokens (6144 -> 5120) ran as 32 launch pairs of
 // the 64-token form, each reading all of W_o: 1023 us; as 256 tiles of
-// 128 x 320 in one launch: 137.  181 tokens: Q/K/V 133 -> 71 us (56 tiles of
-// 256 x 256 before, 168 of 64 x 256 now), O-projection 102 -> 35.
+// 128 x 320 in one launch: 137.  181 tokens: Q/K/V 133 -> 65 us (56 tiles of
+// 256 x 256 before, 224 of 128 x 256 over two splits now), O-projection
+// 102 -> 35.
 //
 // Main loop.  Eight waves in a WM x (8 / WM) grid, v_mfma_f32_16x16x32_f16
 // with W rows as A and tokens as B.  K goes in chunks of 64 through S LDS

@@ -429,12 +429,25 @@ __global__ __launch_bounds__(64 * WAVES) void mq_kernel(MultiQueryArgs a) {
                     const float inv = 1.0f / lt;
                     const size_t tq = static_cast<size_t>(cu.tok + cu.tile * Q + iq[t]);
                     uint16_t *orow = a.out + (tq * nh + cu.h * G + gq[t]) * kHeadDim;
-                    const uint16_t *grow = a.gate ? a.gate + tq * a.gate_stride + (cu.h * G + gq[t]) * kHeadDim : nullptr;
+                    if (a.gate) {
+                        // All of the row's gate requested before any is used.
+                        const uint16_t *grow = a.gate + tq * a.gate_stride + (cu.h * G + gq[t]) * kHeadDim + 4 * grp;
+                        uint2 gw[16];
 #pragma unroll
-                    for (int dt = 0; dt < 16; ++dt)
-                        *reinterpret_cast<uint2 *>(orow + 16 * dt + 4 * grp) =
-                            out_fp16x4(acc[t][dt][0] * inv, acc[t][dt][1] * inv, acc[t][dt][2] * inv,
-                                       acc[t][dt][3] * inv, grow ? grow + 16 * dt + 4 * grp : nullptr);
+                        for (int dt = 0; dt < 16; ++dt) gw[dt] = ld8(grow + 16 * dt);
+#pragma unroll
+                        for (int dt = 0; dt < 16; ++dt)
+                            *reinterpret_cast<uint2 *>(orow + 16 * dt + 4 * grp) =
+                                gate4(pack_out4(acc[t][dt][0] * inv, acc[t][dt][1] * inv, acc[t][dt][2] * inv,
+                                                acc[t][dt][3] * inv),
+                                      gw[dt]);
+                    } else {
+#pragma unroll
+                        for (int dt = 0; dt < 16; ++dt)
+                            *reinterpret_cast<uint2 *>(orow + 16 * dt + 4 * grp) =
+                                pack_out4(acc[t][dt][0] * inv, acc[t][dt][1] * inv, acc[t][dt][2] * inv,
+                                          acc[t][dt][3] * inv);
+                    }
                 }
             } else {
                 // Slot 2w: the unit began at or before this share (its first
