@@ -621,137 +621,209 @@ __global__ __launch_bounds__(64 * kMfmaWaves) void decode_mfma_kernel(DecodeArgs
     }
 }
 
-// Merge the partials of one (sequence, kv head, query head of the group)
-// whose pages were cut across workgroups: 64 lanes x 4 dims per wave.  A
-// separate launch (stream order makes the partials visible), so no
-// cross-workgroup fences are needed: an agent-scope release on every decode
-// workgroup costs an L2 writeback per workgroup on multi-XCD parts.  The
-// (m, l) pairs and acc rows of up to kChunk partials are all requested before
-// any is used, so a sequence cut into at most kChunk pieces costs one memory
-// round trip when the host passes each sequence's first piece and piece
-// count with the launch arguments (DecodeArgs::crec), two otherwise (its
-// length, then its partials).  A sequence cut into more pieces (one long
-// sequence over every CU) has its chunks dealt to the four waves of its
-// workgroup, which merge through LDS.
-//
-// kHeads (the host has shown that no sequence of the launch has more than
-// kChunk pieces): a workgroup per (sequence, kv head), its G waves one
-// query head each, where the general form has a workgroup of four waves per
-// query head.
-constexpr int kCombineWaves = 4;
-template <int G, bool kHeads = false>
-__global__ __launch_bounds__(64 * (kHeads ? G : kCombineWaves)) void combine_kernel(DecodeArgs a) {
+// Where a cut sequence's partials lie: n pieces from workgroups w0 .. w0+n-1.
+// Piece i is in slot 2w when the sequence began at or before that
+// workgroup's range, else 2w+1.  Only w0's range can begin after the
+// sequence's first page, so one division settles every slot (one per piece
+// kept the pieces' loads from going out together).
+struct Pieces {
+    int w0, n, slot0;
+};
+
+// Sequence b's pieces; false when one workgroup covered the sequence and
+// wrote it.  The host passes these with the launch arguments for steps of up
+// to kCombineRecs sequences (DecodeArgs::crec), so a merge's first loads are
+// the partials; otherwise they wait for the sequence's length.
+__device__ __forceinline__ bool find_pieces(const DecodeArgs &a, int b, Pieces &p) {
+    if (a.n_crec > 0) {
+        p.w0 = a.crec[b];
+        if (p.w0 < 0) return false;
+        p.n = a.crec_n[b] >> 1;
+        p.slot0 = 2 * p.w0 + (a.crec_n[b] & 1);
+        return true;
+    }
+    int P, W;
+    stream_k_shape(a, P, W);
+    const int ctx = a.ctx_lens ? a.ctx_lens[b] : a.ctx_len_const;
+    const int npg = (ctx + 15) >> 4;
+    if (npg == 0) return false;
+    const int first = seq_page_base(a, b, npg);
+    p.w0 = wg_of_page<true>(first, P, W);
+    const int w1 = wg_of_page<true>(first + npg - 1, P, W);
+    if (p.w0 == w1) return false;
+    p.n = w1 - p.w0 + 1;
+    p.slot0 = 2 * p.w0 + (first <= wg_start<true>(p.w0, P, W) ? 0 : 1);
+    return true;
+}
+
+// Row of piece i of query head g of kv head h in the partial slots.
+template <int G>
+__device__ __forceinline__ size_t piece_row(const DecodeArgs &a, const Pieces &p, int i, int h, int g) {
+    const int slot = i == 0 ? p.slot0 : 2 * (p.w0 + i);
+    return (static_cast<size_t>(slot) * a.num_kv_heads + h) * G + g;
+}
+
+// Dims d0 .. d0+3 of the merge of at most kCombineChunk pieces by one wave,
+// every load requested before any is used; lt: the sum of probabilities.
+// Both combine forms merge such a sequence here, so a recorded step (always
+// the wide form) gives the bits of the ordinary one.
+template <int G>
+__device__ __forceinline__ float4_t merge_few(const DecodeArgs &a, const Pieces &p, int h, int g, int d0, int lane,
+                                              float &lt) {
     constexpr int kChunk = kCombineChunk;
-    __shared__ float4 w_acc[kCombineWaves * 64];
-    __shared__ float w_ml[kCombineWaves * 2];
+    float2 ml = make_float2(-INFINITY, 0.0f);
+    if (lane < p.n) ml = *reinterpret_cast<const float2 *>(a.ws_ml + piece_row<G>(a, p, lane, h, g) * 2);
+    float4_t v[kChunk];
+#pragma unroll
+    for (int k = 0; k < kChunk; ++k)
+        v[k] = k < p.n ? *reinterpret_cast<const float4_t *>(a.ws_acc + piece_row<G>(a, p, k, h, g) * kHeadDim + d0)
+                       : float4_t{0.f, 0.f, 0.f, 0.f};
+    float cm = ml.x;
+#pragma unroll
+    for (int o = 8; o >= 1; o >>= 1) cm = fmaxf(cm, __shfl_xor(cm, o));
+    cm = __shfl(cm, 0);
+    const float ci = lane < p.n ? __builtin_amdgcn_exp2f(ml.x - cm) : 0.0f;
+    float ls = ci * ml.y;
+#pragma unroll
+    for (int o = 8; o >= 1; o >>= 1) ls += __shfl_xor(ls, o);
+    lt = __shfl(ls, 0);
+    float4_t at = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < kChunk; ++k) {
+        const float ck = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ci), k));
+        at += ck * v[k];
+    }
+    return at;
+}
+
+// Merge the partials of the sequences whose pages were cut across
+// workgroups.  A separate launch (stream order makes the partials visible),
+// so no cross-workgroup fences are needed: an agent-scope release on every
+// decode workgroup costs an L2 writeback per workgroup on multi-XCD parts.
+//
+// combine_kernel (the host has shown that no sequence of the launch has more
+// than kCombineChunk pieces): a workgroup per (sequence, kv head), its G
+// waves one query head each, 64 lanes x 4 dims.  Every (m, l) pair and acc
+// row is requested before any is used, so a merge costs one memory round
+// trip when the pieces come with the arguments, two otherwise.
+template <int G>
+__global__ __launch_bounds__(64 * G) void combine_kernel(DecodeArgs a) {
     const int u = blockIdx.x;
-    const int g = kHeads ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : static_cast<int>(blockIdx.y);
+    const int g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int hkv = a.num_kv_heads;
     const int b = u / hkv;
     const int h = u - b * hkv;
     const int lane = threadIdx.x & 63;
-    const int wave = kHeads ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    // Partial i comes from workgroup w0 + i: slot 2w when the sequence began
-    // at or before that workgroup's range, else 2w+1.  Only w0's range can
-    // begin after the sequence's first page, so one division settles every
-    // slot (one per piece kept the pieces' loads from going out together).
-    int w0, n, slot0;
-    if (a.n_crec > 0) {  // the host's figures, with the kernel arguments
-        w0 = a.crec[b];
-        if (w0 < 0) return;  // one workgroup covered the sequence and wrote it
-        n = a.crec_n[b] >> 1;
-        slot0 = 2 * w0 + (a.crec_n[b] & 1);
-    } else {
-        int P, W;
-        stream_k_shape(a, P, W);
-        const int ctx = a.ctx_lens ? a.ctx_lens[b] : a.ctx_len_const;
-        const int npg = (ctx + 15) >> 4;
-        if (npg == 0) return;
-        const int first = seq_page_base(a, b, npg);
-        w0 = wg_of_page<true>(first, P, W);
-        const int w1 = wg_of_page<true>(first + npg - 1, P, W);
-        if (w0 == w1) return;  // one workgroup covered the sequence and wrote it
-        n = w1 - w0 + 1;
-        slot0 = 2 * w0 + (first <= wg_start<true>(w0, P, W) ? 0 : 1);
-    }
-    const int nw = kHeads ? 1 : blockDim.x >> 6;  // 1 when the host knows no sequence has more than kChunk pieces
-    const bool multi = n > kChunk;   // uniform over the workgroup
-    if (!multi && wave != 0) return;
-    auto row_of = [&](int i) -> size_t {
-        const int slot = i == 0 ? slot0 : 2 * (w0 + i);
-        return (static_cast<size_t>(slot) * hkv + h) * G + g;
+    Pieces p;
+    if (!find_pieces(a, b, p)) return;
+    const uint16_t *gp = gate_of(a, b, h * G + g, lane);
+    const uint2 gw = gp ? ld8(gp) : make_uint2(0, 0);
+    float lt;
+    const float4_t at = merge_few<G>(a, p, h, g, 4 * lane, lane, lt);
+    const float inv = 1.0f / lt;
+    uint2 y = pack_out4(at[0] * inv, at[1] * inv, at[2] * inv, at[3] * inv);
+    if (gp) y = gate4(y, gw);
+    *reinterpret_cast<uint2 *>(a.out + (static_cast<size_t>(b) * a.num_heads + h * G + g) * kHeadDim + 4 * lane) = y;
+}
+
+// combine_wide_kernel (any number of pieces: one long sequence over every CU
+// has 256): a workgroup per (sequence, query head, quarter of the head's
+// dims).  A wave takes four pieces per load instruction, 16 lanes x 4 dims
+// each, and kDepth such loads before it uses any, so NW = 16 waves hold 256
+// pieces in flight at once; lane groups merge by shuffles and waves through
+// LDS.  Latency bounds it: with the whole head in four waves of one
+// workgroup, 16 pieces a wave at a time, 256 pieces took 9.0 us.
+template <int G, int NW>
+__global__ __launch_bounds__(64 * NW) void combine_wide_kernel(DecodeArgs a) {
+    constexpr int kDepth = 4;
+    __shared__ float4 w_acc[NW * 16];
+    __shared__ float2 w_ml[NW];
+    const int u = blockIdx.x;
+    const int g = blockIdx.y;
+    const int hkv = a.num_kv_heads;
+    const int b = u / hkv;
+    const int h = u - b * hkv;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int sub = lane >> 4;                            // piece of the wave's four
+    const int d0 = 64 * blockIdx.z + 4 * (lane & 15);     // this lane's dims
+    Pieces p;
+    if (!find_pieces(a, b, p)) return;  // uniform over the workgroup
+    auto store = [&](const float4_t &o, float l) {
+        const float inv = 1.0f / l;
+        const uint16_t *gp =
+            a.gate ? a.gate + static_cast<int64_t>(b) * a.gate_stride + (h * G + g) * kHeadDim + d0 : nullptr;
+        *reinterpret_cast<uint2 *>(a.out + (static_cast<size_t>(b) * a.num_heads + h * G + g) * kHeadDim + d0) =
+            out_fp16x4(o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv, gp);
     };
-    // Running merge over this wave's chunks: (big, lt, at) is the merge of
-    // the chunks so far (big = -inf, lt = 0 before any).
+    if (p.n <= kCombineChunk) {
+        if (wave != 0) return;
+        float l;
+        const float4_t o = merge_few<G>(a, p, h, g, d0, lane, l);
+        if (lane < 16) store(o, l);
+        return;
+    }
     float big = -INFINITY, lt = 0.0f;
-    float4 at = make_float4(0.f, 0.f, 0.f, 0.f);
-    const int step = multi ? nw * kChunk : kChunk;
-    for (int c0 = (multi ? wave : 0) * kChunk; c0 < n; c0 += step) {
-        const int cnt = min(kChunk, n - c0);
-        float2 ml = make_float2(-INFINITY, 0.0f);
-        if (lane < cnt) ml = *reinterpret_cast<const float2 *>(a.ws_ml + row_of(c0 + lane) * 2);
-        float4 v[kChunk];
+    float4_t at = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int i0 = 4 * wave; i0 < p.n; i0 += 4 * NW * kDepth) {
+        float2 ml[kDepth];
+        float4_t v[kDepth];
 #pragma unroll
-        for (int k = 0; k < kChunk; ++k)
-            v[k] = k < cnt ? reinterpret_cast<const float4 *>(a.ws_acc + row_of(c0 + k) * kHeadDim)[lane]
-                           : make_float4(0.f, 0.f, 0.f, 0.f);
-        float cm = ml.x;
-#pragma unroll
-        for (int o = 8; o >= 1; o >>= 1) cm = fmaxf(cm, __shfl_xor(cm, o));
-        cm = __shfl(cm, 0);
-        const float nb = fmaxf(big, cm);
-        const float keep = __builtin_amdgcn_exp2f(big - nb);  // 0 on the first chunk
-        const float ci = lane < cnt ? __builtin_amdgcn_exp2f(ml.x - nb) : 0.0f;
-        float ls = ci * ml.y;
-#pragma unroll
-        for (int o = 8; o >= 1; o >>= 1) ls += __shfl_xor(ls, o);
-        lt = lt * keep + __shfl(ls, 0);
-        at.x *= keep;
-        at.y *= keep;
-        at.z *= keep;
-        at.w *= keep;
-#pragma unroll
-        for (int k = 0; k < kChunk; ++k) {
-            const float ck = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ci), k));
-            at.x += ck * v[k].x;
-            at.y += ck * v[k].y;
-            at.z += ck * v[k].z;
-            at.w += ck * v[k].w;
+        for (int k = 0; k < kDepth; ++k) {
+            const int i = i0 + 4 * NW * k + sub;
+            const bool ok = i < p.n;
+            const size_t row = piece_row<G>(a, p, ok ? i : 0, h, g);
+            ml[k] = *reinterpret_cast<const float2 *>(a.ws_ml + row * 2);
+            v[k] = *reinterpret_cast<const float4_t *>(a.ws_acc + row * kHeadDim + d0);
+            if (!ok) ml[k].x = -INFINITY;
         }
+        float nb = big;
+#pragma unroll
+        for (int k = 0; k < kDepth; ++k) nb = fmaxf(nb, ml[k].x);
+        if (nb > -INFINITY) {  // this lane group has a piece
+            const float keep = __builtin_amdgcn_exp2f(big - nb);  // 0 before any
+            lt *= keep;
+            at *= keep;
+#pragma unroll
+            for (int k = 0; k < kDepth; ++k) {
+                const float c = __builtin_amdgcn_exp2f(ml[k].x - nb);  // 0 past the last piece
+                lt += c * ml[k].y;
+                at += c * v[k];
+            }
+            big = nb;
+        }
+    }
+    // The four lane groups, then the waves.
+#pragma unroll
+    for (int o = 16; o <= 32; o <<= 1) {
+        const float ob = __shfl_xor(big, o), ol = __shfl_xor(lt, o);
+        float4_t oa;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) oa[c] = __shfl_xor(at[c], o);
+        const float nb = fmaxf(big, ob);
+        const float mu = nb == -INFINITY ? 0.0f : nb;
+        const float c0 = __builtin_amdgcn_exp2f(big - mu), c1 = __builtin_amdgcn_exp2f(ob - mu);
+        lt = lt * c0 + ol * c1;
+        at = at * c0 + oa * c1;
         big = nb;
     }
-    if (multi && nw > 1) {
-        // Wave 0 always holds a chunk; a wave without one (fewer than nw
-        // chunks) keeps big = -inf and weighs 0.
-        w_acc[wave * 64 + lane] = at;
-        if (lane == 0) {
-            w_ml[wave * 2] = big;
-            w_ml[wave * 2 + 1] = lt;
-        }
-        __syncthreads();
-        if (wave != 0) return;
-        float mm = -INFINITY;
+    if (lane < 16) w_acc[wave * 16 + lane] = make_float4(at[0], at[1], at[2], at[3]);
+    if (lane == 0) w_ml[wave] = make_float2(big, lt);
+    __syncthreads();
+    if (threadIdx.x >= 16) return;
+    float mm = -INFINITY;
 #pragma unroll
-        for (int v = 0; v < kCombineWaves; ++v)
-            if (v < nw) mm = fmaxf(mm, w_ml[v * 2]);
-        lt = 0.0f;
-        at = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int w = 0; w < NW; ++w) mm = fmaxf(mm, w_ml[w].x);
+    lt = 0.0f;
+    at = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int v = 0; v < kCombineWaves; ++v) {
-            if (v >= nw) break;
-            const float c = __builtin_amdgcn_exp2f(w_ml[v * 2] - mm);  // 0 for a wave without chunks
-            const float4 x = w_acc[v * 64 + lane];
-            lt += w_ml[v * 2 + 1] * c;
-            at.x += x.x * c;
-            at.y += x.y * c;
-            at.z += x.z * c;
-            at.w += x.w * c;
-        }
+    for (int w = 0; w < NW; ++w) {
+        const float c = __builtin_amdgcn_exp2f(w_ml[w].x - mm);  // 0 for a wave without pieces
+        const float4 x = w_acc[w * 16 + lane];
+        lt += w_ml[w].y * c;
+        at += c * float4_t{x.x, x.y, x.z, x.w};
     }
-    const float inv = 1.0f / lt;
-    *reinterpret_cast<uint2 *>(a.out + (static_cast<size_t>(b) * a.num_heads + h * G + g) * kHeadDim +
-                               4 * lane) =
-        out_fp16x4(at.x * inv, at.y * inv, at.z * inv, at.w * inv, gate_of(a, b, h * G + g, lane));
+    store(at, lt);
 }
 
 // Whole-sequence decode for steps of short sequences: a workgroup walks one
@@ -1051,11 +1123,14 @@ hipError_t launch_g(const DecodeArgs &a, hipStream_t s) {
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(decode_mfma_kernel<G>, dim3(a.n_wg, a.num_kv_heads / hpw), dim3(64 * hpw), 0, s, a);
     if ((e = hipGetLastError()) != hipSuccess || (e = mark(a.ev_after, s)) != hipSuccess) return e;
-    if (a.combine_waves == 1)
-        hipLaunchKernelGGL((combine_kernel<G, true>), dim3(a.n_seqs * a.num_kv_heads), dim3(64 * G), 0, s, a);
+    const int units = a.n_seqs * a.num_kv_heads;
+    // Sixteen waves per workgroup while all of them fit the chip at once.
+    if (a.few_pieces)
+        hipLaunchKernelGGL((combine_kernel<G>), dim3(units), dim3(64 * G), 0, s, a);
+    else if (units * G * 4 <= 512)
+        hipLaunchKernelGGL((combine_wide_kernel<G, 16>), dim3(units, G, 4), dim3(64 * 16), 0, s, a);
     else
-        hipLaunchKernelGGL((combine_kernel<G>), dim3(a.n_seqs * a.num_kv_heads, G), dim3(64 * kCombineWaves), 0, s,
-                           a);
+        hipLaunchKernelGGL((combine_wide_kernel<G, 4>), dim3(units, G, 4), dim3(64 * 4), 0, s, a);
     return hipGetLastError();
 }
 

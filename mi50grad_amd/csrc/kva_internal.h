@@ -157,11 +157,9 @@ struct DecodeArgs {
     int32_t dyn;
     int32_t split_tokens;     // 0 = one workgroup per CU up to the cap
     int32_t min_pages;
-    // 1 (the host has shown that no sequence is cut into more than
-    // kCombineChunk pieces): the combine launch has a workgroup per
-    // (sequence, kv head) with a wave per query head; else a workgroup of
-    // four waves per (sequence, kv head, query head).
-    int32_t combine_waves;
+    // 1: the host has shown that no sequence is cut into more than
+    // kCombineChunk pieces (combine_kernel; else combine_wide_kernel).
+    int32_t few_pieces;
     // The combine's view of each sequence, in the kernel arguments so its
     // first loads are the partials (n_crec = n_seqs <= kCombineRecs; 0: it
     // reads the length from the step plan and derives these): crec[b] = the
