@@ -225,6 +225,11 @@ __device__ __forceinline__ uint4 ld16(const uint16_t *p) {
 __device__ __forceinline__ uint2 ld8(const uint16_t *p) {
     return *reinterpret_cast<const uint2 *>(p);
 }
+// Sixteen bytes at an 8-byte aligned address (a gate row's).
+__device__ __forceinline__ uint4 ld16g(const uint16_t *p) {
+    const uint2 lo = ld8(p), hi = ld8(p + 4);
+    return make_uint4(lo.x, lo.y, hi.x, hi.y);
+}
 __device__ __forceinline__ void st16(uint16_t *p, uint4 v) {
     *reinterpret_cast<uint4 *>(p) = v;
 }

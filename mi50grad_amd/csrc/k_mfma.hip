@@ -11,9 +11,13 @@
 //
 // Unit = (sequence, tile of Q new tokens, kv head).  The tile's query rows
 // are the Q x G (token, query head) pairs of the GQA group packed row after
-// row — every head of the group attends to the same K/V — so four waves of
-// 16 x NT rows each (Q = 64*NT/G) leave at most G-1 rows idle (the tree
-// verify's 9 nodes x 6 heads fill 54 of 64 rows).  Work is split stream-K
+// row — every head of the group attends to the same K/V — so W waves of
+// 16 x NT rows each (Q = 16*W*NT/G) leave at most G-1 rows idle (the tree
+// verify's 9 nodes x 6 heads fill 54 of 64 rows).  Two tiles per wave (256
+// rows a unit) halve the LDS reads per product: the LDS pipe carries K and V
+// once per wave, and with one tile it is as busy as the matrix pipe.  They
+// also double a cut unit's partials, so only steps with enough keys per
+// workgroup take them (mq_two_tiles).  Work is split stream-K
 // over key blocks (64 keys for prefill steps of eight-wave tiles, 32
 // otherwise: mq_keys_for): the blocks of all units are laid end to end, head-major
 // (kv head, sequence, tile), and each workgroup takes an equal share, the
@@ -54,6 +58,7 @@ constexpr int kPairBytes = 2 * kRowBytes + 32;      // two keys, then 32 B of pa
 template <int KEYS> constexpr int ring_stages() { return KEYS == 32 ? 4 : 2; }
 template <int KEYS> constexpr int tile_bytes() { return KEYS / 2 * kPairBytes; }  // K or V of a block
 constexpr float kLog2e = 1.4426950408889634f;
+constexpr int kStripRow = 128 + 16;  // a row of a wave's epilogue strip: 64 dims, padded
 
 
 __device__ __forceinline__ int mq_wg_start(int w, int n, int W) { return floor_muldiv(w, n, W); }
@@ -108,7 +113,7 @@ template <int KEYS>
 __device__ __forceinline__ Unit load_unit(const MultiQueryArgs &a, int u, int b) {
     Unit x;
     x.u = u;
-    x.ub = ld_uniform(a.mq_pre + u) + mq_unit_cost(KEYS);  // its first block (positions before: the start cost)
+    x.ub = ld_uniform(a.mq_pre + u) + kMqUnitCost;  // its first block (positions before: the start cost)
     x.ue = ld_uniform(a.mq_pre + u + 1);
     const int U1 = ld_uniform(a.upre + a.n_seqs);
     x.h = u / U1;
@@ -152,11 +157,25 @@ __device__ __forceinline__ void issue_block(uint8_t *st, const MultiQueryArgs &a
     const uint32_t n = on ? kBlockTokens * row_bytes : 0u;
     const auto rk = ro_rsrc(a.k_pool + off, n), rv = ro_rsrc(a.v_pool + off, n);
     const int q = lane & 31;
+    if (key0 + kPer - 1 <= last) {
+        // All of the wave's keys exist (the sequence's last block aside):
+        // rows two apart differ by a scalar offset.
+        const int row0 = (key0 & 15) + (lane >> 5);
+        const int kl = lane >> 5;  // parity of the key (kPer is even)
+        const uint32_t vk = row0 * row_bytes + 16 * k_granule(kl, q), vv = row0 * row_bytes + 16 * v_granule(kl, q);
+#pragma unroll
+        for (int i = 0; i < kPer / 2; ++i) {
+            const uint32_t dst = lds_addr(st + (kPer * wv / 2 + i) * kPairBytes);  // this load's two keys
+            load_to_lds_at(rk, dst, vk, 2 * i * row_bytes);
+            load_to_lds_at(rv, dst + tile_bytes<KEYS>(), vv, 2 * i * row_bytes);
+        }
+        return;
+    }
 #pragma unroll
     for (int i = 0; i < kPer / 2; ++i) {
         const int kl = kPer * wv + 2 * i + (lane >> 5);  // key within the block
         const int row = min(key0 + 2 * i + (lane >> 5), last) & 15;
-        const uint32_t dst = lds_addr(st + (kPer * wv / 2 + i) * kPairBytes);  // this load's two keys
+        const uint32_t dst = lds_addr(st + (kPer * wv / 2 + i) * kPairBytes);
         load_to_lds(rk, dst, row * row_bytes + 16 * k_granule(kl, q));
         load_to_lds(rv, dst + tile_bytes<KEYS>(), row * row_bytes + 16 * v_granule(kl, q));
     }
@@ -185,13 +204,27 @@ __device__ __forceinline__ int mq_share_of(int i, int W) {
     return (W & 7) == 0 ? (i & 7) * (W >> 3) + (i >> 3) : i;
 }
 
+// Operands read ahead of the products that use them.  Left alone, the
+// compiler reads one operand, waits for it and multiplies: an LDS round trip
+// (over 100 cycles) for every 16 to 32 cycles of products.  The scheduling
+// barriers pin the order; a ring of operands holds the reads in flight.
+// Two tiles per wave, 2048 tokens after 16400: 886 us unpinned, 798 with three
+// ahead, 808 with two and 813 with four (more registers than there are); one
+// tile per wave 1050 -> 959.
+constexpr int kQkAhead = 3, kPvAhead = 3;
+
 template <int NT, int WAVES, bool TREE, int KEYS>
 __global__ __launch_bounds__(64 * WAVES) void mq_kernel(MultiQueryArgs a) {
     constexpr int kRing = ring_stages<KEYS>();
     constexpr int kTileBytes = tile_bytes<KEYS>();
-    constexpr int kKT = KEYS / 16;  // 16-key tiles of a block (QK)
-    constexpr int kKS = KEYS / 32;  // 32-key steps of a block (PV)
+    // Keys folded in at a time: a block's, or with two row tiles per wave
+    // half of a 64-key block's (the scores of all would not fit the
+    // registers beside two tiles' accumulators).
+    constexpr int kFold = NT == 1 ? KEYS : 32;
+    constexpr int kKT = kFold / 16;  // 16-key tiles of a fold (QK)
+    constexpr int kKS = kFold / 32;  // 32-key steps of a fold (PV)
     __shared__ __attribute__((aligned(16))) uint8_t ring[kRing][2 * kTileBytes];
+    __shared__ __attribute__((aligned(16))) uint8_t strips[WAVES][16 * kStripRow];  // the epilogue's, per wave
     const int w = mq_share_of(blockIdx.x, a.n_wg);  // this workgroup's share (and partial slots)
     const int W = a.n_wg;
     const int NB = a.total_blocks;
@@ -209,13 +242,12 @@ __global__ __launch_bounds__(64 * WAVES) void mq_kernel(MultiQueryArgs a) {
     const int row_bytes = hkv * kRowBytes;
     const float scale = kLog2e / 16.0f;
 
-    // This lane's query row in each of the wave's NT tiles: (token iq, head gq).
-    int iq[NT], gq[NT];
+    // The token of this lane's query row in each of the wave's NT tiles.
+    int iq[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
         const int rho = 16 * (wv * NT + t) + col;
         iq[t] = rho / G;
-        gq[t] = rho - iq[t] * G;
     }
 
     // Issue side: the unit and block of the next load, kRing-1 blocks ahead
@@ -227,6 +259,18 @@ __global__ __launch_bounds__(64 * WAVES) void mq_kernel(MultiQueryArgs a) {
     if (ig >= q1) return;  // the share holds only a unit's start cost
     int ipage = 0;  // page of the next issue
     auto fetch_page = [&]() { ipage = block_page<WAVES, KEYS>(iu, ig, ig < q1, wv); };
+    // With two stages every load has landed when a block begins, so the
+    // page of the next issue can come by a vector load behind this block's:
+    // no wait of its own (a scalar load ahead of its use would make every
+    // LDS wait of the block drain, scalar loads returning out of order).
+    constexpr bool kPageAhead = kRing == 2;
+    int vpage = 0;
+    auto page_ahead = [&]() {
+        const int key0 = (ig - iu.ub) * KEYS + KEYS / WAVES * wv;
+        const auto tr = ro_rsrc(iu.trow, static_cast<uint32_t>(a.table_stride) * 4u);
+        vpage = static_cast<int>(
+            __builtin_amdgcn_raw_buffer_load_b32(tr, ig < q1 ? 4 * (min(key0, iu.ctx - 1) >> 4) : 0, 0, 0));
+    };
     auto issue = [&](int slot) {
         const bool on = ig < q1;
         issue_block<WAVES, KEYS>(ring[slot], a, iu, ig, on, ipage, wv, lane, row_bytes);
@@ -242,12 +286,17 @@ __global__ __launch_bounds__(64 * WAVES) void mq_kernel(MultiQueryArgs a) {
         fetch_page();
         issue(s);
     }
+    if constexpr (kPageAhead) page_ahead();
 
     int n_done = 0;  // blocks computed by this workgroup (ring position)
     while (true) {
         const int seg_end = min(cu.ue, q1);
         const bool whole = g == cu.ub && seg_end == cu.ue;
-        // Query rows of this unit.
+        // Query rows of this unit.  Four lanes load 64 contiguous bytes of a
+        // row (in the operand layout's lane order, a load's 64 lanes touch
+        // 16 rows in 16-byte pieces, at a third of the rate), then a lane
+        // permutation gives each lane its operand pieces.  Rows past the
+        // unit's tokens read a row that exists; they are never written.
         bool qvalid[NT];
         int qslot[NT];
         uint64_t qbits[NT];
@@ -258,11 +307,24 @@ __global__ __launch_bounds__(64 * WAVES) void mq_kernel(MultiQueryArgs a) {
             qvalid[t] = iq[t] < Q && qi < cu.T;
             qslot[t] = cu.ns + qi;
             qbits[t] = (TREE && qvalid[t]) ? a.tok_bits[cu.tok + qi] : 0ull;
-            const uint16_t *qr =
-                a.q + (static_cast<size_t>(cu.tok + (qvalid[t] ? qi : 0)) * nh + cu.h * G + gq[t]) * kHeadDim;
+            const int rl = 16 * (wv * NT + t) + (lane >> 2);
+            const int il = rl / G, ql = cu.tile * Q + il;
+            const bool has = il < Q && ql < cu.T;
+            const uint16_t *qr = a.q +
+                                 (static_cast<size_t>(cu.tok + (has ? ql : 0)) * nh + cu.h * G + (has ? rl - il * G : 0)) *
+                                     kHeadDim +
+                                 8 * (lane & 3);
 #pragma unroll
-            for (int kk = 0; kk < 8; ++kk)
-                qb[t][kk] = qvalid[t] ? ld16(qr + 32 * kk + 8 * grp) : make_uint4(0, 0, 0, 0);
+            for (int kk = 0; kk < 8; ++kk) qb[t][kk] = ld16(qr + 32 * kk);
+            const int from = 4 * (4 * col + grp);  // bytes: the lane that holds this lane's pieces
+#pragma unroll
+            for (int kk = 0; kk < 8; ++kk) {
+                qb[t][kk].x = __builtin_amdgcn_ds_bpermute(from, qb[t][kk].x);
+                qb[t][kk].y = __builtin_amdgcn_ds_bpermute(from, qb[t][kk].y);
+                qb[t][kk].z = __builtin_amdgcn_ds_bpermute(from, qb[t][kk].z);
+                qb[t][kk].w = __builtin_amdgcn_ds_bpermute(from, qb[t][kk].w);
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
         // Take delivery of the query rows here, once per unit: left to the
         // compiler, the wait for them would sit inside the block loop and
@@ -288,29 +350,43 @@ __global__ __launch_bounds__(64 * WAVES) void mq_kernel(MultiQueryArgs a) {
             wait_block<WAVES, KEYS>();
             __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_sched_barrier(0);
-            fetch_page();
+            if constexpr (kPageAhead)
+                ipage = __builtin_amdgcn_readfirstlane(vpage);
+            else
+                fetch_page();
             issue((n_done + kRing - 1) % kRing);
+            if constexpr (kPageAhead) page_ahead();
             __builtin_amdgcn_sched_barrier(0);
-            const uint8_t *kt = ring[n_done % kRing];
+#pragma unroll 1
+            for (int fold = 0; fold < KEYS / kFold; ++fold) {
+            // (The fold's body is not indented a level further.)
+            const uint8_t *kt = ring[n_done % kRing] + fold * (kFold / 2) * kPairBytes;
             const uint8_t *kbase = kt + key_off(col) + 16 * k_granule(col, grp);
-            const int key0 = (g - cu.ub) * KEYS;
+            const int key0 = (g - cu.ub) * KEYS + fold * kFold;
 
             // S^T for keys key0 + 16*nt + 4*grp + i, row `col` of each tile.
             float4_t s[NT][kKT];
 #pragma unroll
-            for (int nt = 0; nt < kKT; ++nt) {
+            for (int nt = 0; nt < kKT; ++nt)
 #pragma unroll
                 for (int t = 0; t < NT; ++t) s[t][nt] = float4_t{0.f, 0.f, 0.f, 0.f};
-                // key 16*nt + col, granule 4*kk + grp: kbase + nt*8 pairs + 64*kk
-                const uint8_t *kr = kbase + 8 * nt * kPairBytes;
+            // Operand i: key tile i % kKT (key 16*nt + col), k-step i / kKT
+            // (granule 4*kk + grp): kbase + nt*8 pairs + 64*kk.
+            auto read_k = [&](int i) -> uint4 {
+                return *reinterpret_cast<const uint4 *>(kbase + 8 * (i % kKT) * kPairBytes + 64 * (i / kKT));
+            };
+            uint4 ka[kQkAhead];
 #pragma unroll
-                for (int kk = 0; kk < 8; ++kk) {
-                    const uint4 ka = *reinterpret_cast<const uint4 *>(kr + 64 * kk);
+            for (int i = 0; i < kQkAhead; ++i) ka[i] = read_k(i);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int t = 0; t < NT; ++t)
-                        s[t][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(ka), as_h8(qb[t][kk]), s[t][nt],
-                                                                        0, 0, 0);
-                }
+            for (int i = 0; i < 8 * kKT; ++i) {
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+                    s[t][i % kKT] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(ka[i % kQkAhead]), as_h8(qb[t][i / kKT]),
+                                                                          s[t][i % kKT], 0, 0, 0);
+                if (i + kQkAhead < 8 * kKT) ka[i % kQkAhead] = read_k(i + kQkAhead);
+                __builtin_amdgcn_sched_barrier(0);
             }
             half8_t pb[NT][kKS];
             float corr[NT];
@@ -319,7 +395,7 @@ __global__ __launch_bounds__(64 * WAVES) void mq_kernel(MultiQueryArgs a) {
             // every row (wave-uniform test); otherwise mask key by key.  Rows
             // past the unit's tokens are never written, so the open case
             // needs no mask at all.
-            const bool open = key0 + KEYS <= cu.ns;
+            const bool open = key0 + kFold <= cu.ns;
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
                 // Masked scores become -inf; the max is taken over the raw
@@ -398,23 +474,32 @@ __global__ __launch_bounds__(64 * WAVES) void mq_kernel(MultiQueryArgs a) {
             const int vs = lane & 3;
             const uint8_t *vb = kt + kTileBytes + key_off(4 * grp + vr) + 16 * (vs >> 1) + 8 * (vs & 1);
             const uint8_t *vbase[2] = {vb + 64 * (vr & 1), vb - 64 * (vr & 1)};
+            // Operand i: dim tile i / kKS, keys 32*(i % kKS) .. (16 pairs on).
+            auto read_v = [&](int i) -> half8_t {
+                short4_t part[2];
 #pragma unroll
-            for (int dt = 0; dt < 16; ++dt) {
-#pragma unroll
-                for (int ks = 0; ks < kKS; ++ks) {  // keys 32*ks ..: 16 pairs on
-                    short4_t part[2];
-#pragma unroll
-                    for (int hh = 0; hh < 2; ++hh) {
-                        const uint8_t *src = vbase[(dt >> 1) & 1] + (16 * ks + 8 * hh) * kPairBytes + 32 * dt;
-                        part[hh] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t *)src);
-                    }
-                    const uint2 v0 = __builtin_bit_cast(uint2, part[0]);
-                    const uint2 v1 = __builtin_bit_cast(uint2, part[1]);
-                    const half8_t va = __builtin_bit_cast(half8_t, make_uint4(v0.x, v0.y, v1.x, v1.y));
-#pragma unroll
-                    for (int t = 0; t < NT; ++t)
-                        acc[t][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pb[t][ks], acc[t][dt], 0, 0, 0);
+                for (int hh = 0; hh < 2; ++hh) {
+                    const uint8_t *src =
+                        vbase[(i / kKS >> 1) & 1] + (16 * (i % kKS) + 8 * hh) * kPairBytes + 32 * (i / kKS);
+                    part[hh] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t *)src);
                 }
+                const uint2 v0 = __builtin_bit_cast(uint2, part[0]);
+                const uint2 v1 = __builtin_bit_cast(uint2, part[1]);
+                return __builtin_bit_cast(half8_t, make_uint4(v0.x, v0.y, v1.x, v1.y));
+            };
+            half8_t va[kPvAhead];
+#pragma unroll
+            for (int i = 0; i < kPvAhead; ++i) va[i] = read_v(i);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 16 * kKS; ++i) {
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+                    acc[t][i / kKS] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va[i % kPvAhead], pb[t][i % kKS],
+                                                                            acc[t][i / kKS], 0, 0, 0);
+                if (i + kPvAhead < 16 * kKS) va[i % kPvAhead] = read_v(i + kPvAhead);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             }
             ++n_done;
         }
@@ -425,29 +510,53 @@ __global__ __launch_bounds__(64 * WAVES) void mq_kernel(MultiQueryArgs a) {
             const float lt = group4_sum(l[t]);
             const int rho = 16 * (wv * NT + t) + col;
             if (whole) {
-                if (qvalid[t]) {
-                    const float inv = 1.0f / lt;
-                    const size_t tq = static_cast<size_t>(cu.tok + cu.tile * Q + iq[t]);
-                    uint16_t *orow = a.out + (tq * nh + cu.h * G + gq[t]) * kHeadDim;
-                    if (a.gate) {
-                        // All of the row's gate requested before any is used.
-                        const uint16_t *grow = a.gate + tq * a.gate_stride + (cu.h * G + gq[t]) * kHeadDim + 4 * grp;
-                        uint2 gw[16];
+                // Through the wave's LDS strip, 64 dims at a time, so that
+                // eight lanes hold 128 contiguous bytes of a row: the gate is
+                // read and the output written in whole lines (from the
+                // accumulator layout, in 32-byte pieces of 16 rows, a unit's
+                // end took 2.2 to 5 us).
+                const float inv = 1.0f / lt;
+                const int r8 = lane >> 3, c8 = lane & 7;  // row (and row + 8) and 16-byte piece
+                bool has[2];
+                size_t orow[2], grow[2];
 #pragma unroll
-                        for (int dt = 0; dt < 16; ++dt) gw[dt] = ld8(grow + 16 * dt);
+                for (int hh = 0; hh < 2; ++hh) {
+                    const int rl = 16 * (wv * NT + t) + 8 * hh + r8;
+                    const int il = rl / G, ql = cu.tile * Q + il;
+                    has[hh] = il < Q && ql < cu.T;
+                    const size_t tq = static_cast<size_t>(cu.tok + (has[hh] ? ql : 0));
+                    const int hq = cu.h * G + (has[hh] ? rl - il * G : 0);
+                    orow[hh] = (tq * nh + hq) * kHeadDim + 8 * c8;
+                    grow[hh] = tq * a.gate_stride + hq * kHeadDim + 8 * c8;
+                }
+                constexpr int kGateAhead = NT == 1 ? 4 : 1;  // strips of gate requested together
+                uint4 gw[kGateAhead][2];
+                uint8_t *strip = strips[wv];
 #pragma unroll
-                        for (int dt = 0; dt < 16; ++dt)
-                            *reinterpret_cast<uint2 *>(orow + 16 * dt + 4 * grp) =
-                                gate4(pack_out4(acc[t][dt][0] * inv, acc[t][dt][1] * inv, acc[t][dt][2] * inv,
-                                                acc[t][dt][3] * inv),
-                                      gw[dt]);
-                    } else {
+                for (int c = 0; c < 4; ++c) {
+                    if (a.gate && c % kGateAhead == 0) {
 #pragma unroll
-                        for (int dt = 0; dt < 16; ++dt)
-                            *reinterpret_cast<uint2 *>(orow + 16 * dt + 4 * grp) =
-                                pack_out4(acc[t][dt][0] * inv, acc[t][dt][1] * inv, acc[t][dt][2] * inv,
-                                          acc[t][dt][3] * inv);
+                        for (int k = 0; k < kGateAhead; ++k)
+#pragma unroll
+                            for (int hh = 0; hh < 2; ++hh) gw[k][hh] = ld16g(a.gate + grow[hh] + 64 * (c + k));
                     }
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) {
+                        const float4_t o = acc[t][4 * c + d] * inv;
+                        *reinterpret_cast<uint2 *>(strip + kStripRow * col + 32 * d + 8 * grp) =
+                            pack_out4(o[0], o[1], o[2], o[3]);
+                    }
+#pragma unroll
+                    for (int hh = 0; hh < 2; ++hh) {
+                        uint4 y = *reinterpret_cast<const uint4 *>(strip + kStripRow * (8 * hh + r8) + 16 * c8);
+                        if (a.gate) {
+                            const uint2 lo = gate4(make_uint2(y.x, y.y), make_uint2(gw[c % kGateAhead][hh].x, gw[c % kGateAhead][hh].y));
+                            const uint2 hi = gate4(make_uint2(y.z, y.w), make_uint2(gw[c % kGateAhead][hh].z, gw[c % kGateAhead][hh].w));
+                            y = make_uint4(lo.x, lo.y, hi.x, hi.y);
+                        }
+                        if (has[hh]) st16(a.out + orow[hh] + 64 * c, y);
+                    }
+                    if (NT > 1) __builtin_amdgcn_sched_barrier(0);
                 }
             } else {
                 // Slot 2w: the unit began at or before this share (its first
@@ -553,7 +662,9 @@ hipError_t launch_mq(const MultiQueryArgs &a, hipStream_t s) {
         const hipError_t e = hipEventRecord(a.ev_before, s);
         if (e != hipSuccess) return e;
     }
-    if (a.tree) {
+    if constexpr (NT > 1) {  // long prefill steps only
+        hipLaunchKernelGGL((mq_kernel<NT, WAVES, false, 64>), dim3(a.n_wg), dim3(64 * WAVES), 0, s, a);
+    } else if (a.tree) {
         hipLaunchKernelGGL((mq_kernel<NT, WAVES, true, 32>), dim3(a.n_wg), dim3(64 * WAVES), 0, s, a);
     } else if (k64) {
         if constexpr (WAVES == 8)
@@ -578,6 +689,7 @@ hipError_t launch_multi_query(const MultiQueryArgs &a, hipStream_t s) {
     if (a.q_tile != mq_tile_tokens(G, a.n_waves, a.n_t)) return hipErrorInvalidValue;
     if (a.n_t == 1 && a.n_waves == 4) return launch_mq<1, 4>(a, s);
     if (a.n_t == 1 && a.n_waves == 8) return launch_mq<1, 8>(a, s);
+    if (a.n_t == 2 && a.n_waves == 8 && a.keys == 64 && !a.tree) return launch_mq<2, 8>(a, s);
     return hipErrorInvalidValue;
 }
 

@@ -117,6 +117,7 @@ struct kva_cache {
     int32_t st_mq_blocks = 0;    // key blocks (and unit start costs) of all multi-query units
     int32_t st_mq_waves = 4;     // waves per workgroup of the multi-query kernel
     int32_t st_mq_keys = 32;     // keys per multi-query block (mq_keys_for)
+    int32_t st_mq_nt = 1;        // 16-row tiles per wave
     int32_t st_mq_q = 0;         // new tokens per unit tile
     size_t off_upre = 0, off_mqpre = 0;
     bool st_all_one = false, st_has_bits = false;
@@ -660,7 +661,16 @@ int kva_step_begin(kva_cache *c, int32_t n_seqs, const int32_t *seq_ids, const i
     int32_t run_max = 0;
     for (int32_t b = 0; b < n_seqs; ++b) run_max = std::max(run_max, n_new[b]);
     const int32_t mq_waves = kva::mq_waves_for(group, run_max);
-    const int32_t mq_q = kva::mq_tile_tokens(group, mq_waves, 1);
+    // Blocks of the step in one-tile units, each tile's keys taken as its
+    // sequence's mean.
+    int64_t one_tile_blocks = 0;
+    for (int32_t b = 0; b < n_seqs; ++b) {
+        const int64_t tiles = (n_new[b] + kva::mq_tile_tokens(group, mq_waves, 1) - 1) / kva::mq_tile_tokens(group, mq_waves, 1);
+        one_tile_blocks += tiles * c->cfg.num_kv_heads * ((c->len[seq_ids[b]] + n_new[b] / 2) / 64 + 1);
+    }
+    const int32_t mq_nt =
+        mq_waves == 8 && !tree_bits && kva::mq_two_tiles(one_tile_blocks, c->mq_max_wg) ? 2 : 1;
+    const int32_t mq_q = kva::mq_tile_tokens(group, mq_waves, mq_nt);
     int64_t n_units = 0;
     for (int32_t b = 0; b < n_seqs; ++b)
         n_units += static_cast<int64_t>((n_new[b] + mq_q - 1) / mq_q) * c->cfg.num_kv_heads;
@@ -742,7 +752,7 @@ int kva_step_begin(kva_cache *c, int32_t n_seqs, const int32_t *seq_ids, const i
     }
     p_upre[n_seqs] = static_cast<int32_t>(tiles_all);
     const int32_t mq_keys = kva::mq_keys_for(mq_waves, tree_bits != nullptr);
-    const int32_t unit_cost = kva::mq_unit_cost(mq_keys);
+    constexpr int32_t unit_cost = kva::kMqUnitCost;
     int64_t units = 0, blocks = 0;
     for (int32_t hh = 0; hh < c->cfg.num_kv_heads; ++hh) {
         for (int32_t b = 0; b < n_seqs; ++b) {
@@ -835,6 +845,7 @@ int kva_step_begin(kva_cache *c, int32_t n_seqs, const int32_t *seq_ids, const i
     c->st_mq_waves = mq_waves;
     c->st_mq_keys = mq_keys;
     c->st_mq_q = mq_q;
+    c->st_mq_nt = mq_nt;
     c->off_upre = o_upre;
     c->off_mqpre = o_mqpre;
     c->st_all_one = all_one;
@@ -1364,7 +1375,7 @@ static int multi_query(kva_cache *c, int32_t layer, const void *q, void *out, kv
     a.num_kv_heads = c->cfg.num_kv_heads;
     a.tree = tree ? 1 : 0;
     a.n_waves = c->st_mq_waves;
-    a.n_t = 1;
+    a.n_t = c->st_mq_nt;
     a.q_tile = c->st_mq_q;
     a.ws_acc = c->d_mq_acc;
     a.ws_ml = c->d_mq_ml;

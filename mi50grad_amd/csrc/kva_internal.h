@@ -251,7 +251,7 @@ struct MultiQueryArgs {
     const int32_t *tok_off;   // device [n_seqs+1]: new-token ranges
     const uint64_t *tok_bits; // device [T] (tree mode) or null
     const int32_t *upre;      // device [n_seqs+1]: tiles of earlier sequences (units of one head)
-    const int32_t *mq_pre;    // device [n_units+1]: positions of earlier units (blocks + mq_unit_cost each)
+    const int32_t *mq_pre;    // device [n_units+1]: positions of earlier units (blocks + kMqUnitCost each)
     // Device [n_cut][kMqCutWords]: the units cut across workgroups, as
     // kva_step_begin found them from the shares of n_wg (head, first new
     // token of the tile, its valid tokens, first and last share, first
@@ -260,14 +260,14 @@ struct MultiQueryArgs {
     int32_t n_cut;
     int32_t n_seqs;
     int32_t n_units;          // (kv head, sequence, token tile) units, head-major
-    int32_t total_blocks;     // positions of all units (blocks + mq_unit_cost each)
+    int32_t total_blocks;     // positions of all units (blocks + kMqUnitCost each)
     int32_t keys;             // keys per block: mq_keys_for(n_waves, the step has tree bits)
     int32_t n_wg;             // workgroups sharing the blocks (stream-K)
     int32_t num_heads;
     int32_t num_kv_heads;
     int32_t tree;             // 0 = causal chunk, 1 = tree mask
     int32_t n_waves;          // waves per workgroup (4 or 8)
-    int32_t n_t;              // 16-row MFMA tiles per wave (1: the form launched)
+    int32_t n_t;              // 16-row MFMA tiles per wave (1 or 2: mq_two_tiles)
     int32_t q_tile;           // new tokens per unit tile: mq_tile_tokens(G, n_waves, n_t)
     float *ws_acc;            // [2*n_wg][kMqSlotRows][256] partial slots
     float *ws_ml;             // [2*n_wg][kMqSlotRows][2]
@@ -285,16 +285,16 @@ struct MultiQueryArgs {
 // (config 5 at 64 keys: 862 -> 888 us) and for small steps.  A step planned
 // with tree bits uses 32 for kva_prefill too.
 constexpr int mq_keys_for(int waves, bool tree_plan) { return (waves == 8 && !tree_plan) ? 64 : 32; }
-// The stream-K split of the multi-query kernel counts each unit as the
-// blocks of 128 more keys than it has (the cost of starting a unit: its
-// query rows, its output), so a share full of short units gets fewer
+// The stream-K split of the multi-query kernel counts each unit as this many
+// blocks more than it has: the cost of starting and ending a unit (its query
+// rows, its gate and output), so a share full of short units gets fewer
 // blocks.  Unit u's blocks sit at positions [mq_pre[u] + cost, mq_pre[u+1]).
-// 128 keys: a unit start measured about two 32-key blocks' time, but with
-// two the shares holding many short units still ended last (config 4 at 32
-// keys per block, cost 2 -> 132 us, 3 -> 122, 4 -> 116, 5 and 6 -> 116-117).
-constexpr int mq_unit_cost(int keys) { return 128 / keys; }
+// Counted as 2, 3, 4 and 5 blocks of 64 keys, 4 x 512 gated tokens after 46
+// to 1655 cached rows took 124, 119, 114 and 121 us; blocks of 32 keys (each
+// half the time, so half the cost would do) 4 as well.
+constexpr int kMqUnitCost = 4;
 constexpr int kMqMaxGroup = 8;    // largest GQA group of the multi-query kernel
-constexpr int kMqSlotRows = 128;  // query rows of a partial slot (waves x 16 x tiles at most)
+constexpr int kMqSlotRows = 256;  // query rows of a partial slot (waves x 16 x tiles at most)
 constexpr int kMqCutWords = 8;    // int32 words of a cut-unit record (6 used)
 // Workgroups of a multi-query launch over `blocks` positions: one per CU (the
 // cap), at least 128 keys' blocks each.  kva_step_begin (the cut-unit
@@ -313,6 +313,13 @@ constexpr int mq_tile_tokens(int G, int n_waves, int n_t) { return 16 * n_waves 
 // SIMD) when a whole run fits one unit of 64 rows (tree verify), else eight
 // (128 rows; two waves per SIMD hide each other's softmax and LDS waits).
 constexpr int mq_waves_for(int G, int max_new) { return max_new * G <= 64 ? 4 : 8; }
+// Whether an eight-wave causal step takes two row tiles per wave: with
+// `blocks` 64-key blocks in one-tile units over `wgs` workgroups.  Two tiles
+// save 15 % of a block's time and cost about 13 us in partials and unit
+// starts: 2048 tokens after 16400 rows (417 blocks a workgroup) 778 + 28 us
+// of combine against 955 + 19, after 4000 (120) 272 + 28 against 308 + 18;
+// 512 after 4000 (26) 83 + 15 against 80 + 11.
+constexpr bool mq_two_tiles(int64_t blocks, int32_t wgs) { return blocks >= 48 * static_cast<int64_t>(wgs); }
 hipError_t launch_multi_query(const MultiQueryArgs &a, hipStream_t s);
 
 }  // namespace kva
