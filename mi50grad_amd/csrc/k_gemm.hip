@@ -20,9 +20,9 @@
 //   whole tiles would leave most of the 256 CUs idle.
 // The O-projection of 2048 tokens (6144 -> 5120) ran as 32 launch pairs of
 // the 64-token form, each reading all of W_o: 1023 us; as 256 tiles of
-// 128 x 320 in one launch: 137.  181 tokens: Q/K/V 133 -> 65 us (56 tiles of
-// 256 x 256 before, 224 of 128 x 256 over two splits now), O-projection
-// 102 -> 35.
+// 128 x 320 in one launch: 137.  181 tokens: Q/K/V 133 -> 52 us (56 tiles of
+// 256 x 256 before, 224 of 192 x 128 over two splits now), O-projection
+// 102 -> 27.
 //
 // Main loop.  Eight waves in a WM x (8 / WM) grid, v_mfma_f32_16x16x32_f16
 // with W rows as A and tokens as B.  K goes in chunks of 64 through S LDS
@@ -377,6 +377,8 @@ using Tile256x256 = GTile<256, 256, 2, 2, 0>;
 using Tile128x256 = GTile<128, 256, 2, 3, 1>;
 using Tile64x256 = GTile<64, 256, 1, 3, 1>;
 using Tile128x320 = GTile<128, 320, 2, 2, 1>;
+using Tile256x128 = GTile<256, 128, 4, 3, 1>;
+using Tile192x128 = GTile<192, 128, 4, 3, 1>;
 using Tile128x128 = GTile<128, 128, 2, 4, 1>;
 using Tile64x128 = GTile<64, 128, 1, 6, 1>;
 
@@ -404,6 +406,8 @@ const GemmForm kForms[] = {
      launch_gemm<Tile128x256, kEpiPart>},
     {64, 256, 0.84f, true, false, true, launch_gemm<Tile64x256, kEpiHead>, nullptr, launch_gemm<Tile64x256, kEpiPart>},
     {128, 320, 1.30f, false, true, false, nullptr, launch_gemm<Tile128x320, kEpiOut>, nullptr},
+    {256, 128, 0.96f, false, true, true, nullptr, launch_gemm<Tile256x128, kEpiOut>, launch_gemm<Tile256x128, kEpiPart>},
+    {192, 128, 0.76f, false, true, true, nullptr, launch_gemm<Tile192x128, kEpiOut>, launch_gemm<Tile192x128, kEpiPart>},
     {128, 128, 0.64f, false, true, true, nullptr, launch_gemm<Tile128x128, kEpiOut>, launch_gemm<Tile128x128, kEpiPart>},
     {64, 128, 0.47f, false, true, true, nullptr, launch_gemm<Tile64x128, kEpiOut>, launch_gemm<Tile64x128, kEpiPart>},
 };
@@ -415,8 +419,10 @@ const GemmForm kForms[] = {
 // estimate is within 15 % of the measured times it was fitted to (64 to 2048
 // tokens of 5120 -> 14336 and 6144 -> 5120, and their halves and quarters):
 // 2048 tokens of 6144 -> 5120 take 137 us in 128 x 320 tiles (one round of
-// 256), 202 in 128 x 256 (two rounds of 320); 181 take 29 us in 128 x 128
-// over three splits, 69 unsplit.
+// 256), 202 in 128 x 256 (two rounds of 320); 181 take 22 us in 192 x 128
+// over six splits, 29 in 128 x 128 over three, 69 unsplit, and their Q/K/V 46
+// us in 192 x 128 over two splits against 59 in 128 x 256 (a tile that holds
+// every token reads each weight row once).
 struct GemmPlan {
     const GemmForm *form;
     int splits;

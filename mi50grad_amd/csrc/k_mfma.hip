@@ -359,147 +359,146 @@ __global__ __launch_bounds__(64 * WAVES) void mq_kernel(MultiQueryArgs a) {
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll 1
             for (int fold = 0; fold < KEYS / kFold; ++fold) {
-            // (The fold's body is not indented a level further.)
-            const uint8_t *kt = ring[n_done % kRing] + fold * (kFold / 2) * kPairBytes;
-            const uint8_t *kbase = kt + key_off(col) + 16 * k_granule(col, grp);
-            const int key0 = (g - cu.ub) * KEYS + fold * kFold;
+                const uint8_t *kt = ring[n_done % kRing] + fold * (kFold / 2) * kPairBytes;
+                const uint8_t *kbase = kt + key_off(col) + 16 * k_granule(col, grp);
+                const int key0 = (g - cu.ub) * KEYS + fold * kFold;
 
-            // S^T for keys key0 + 16*nt + 4*grp + i, row `col` of each tile.
-            float4_t s[NT][kKT];
-#pragma unroll
-            for (int nt = 0; nt < kKT; ++nt)
-#pragma unroll
-                for (int t = 0; t < NT; ++t) s[t][nt] = float4_t{0.f, 0.f, 0.f, 0.f};
-            // Operand i: key tile i % kKT (key 16*nt + col), k-step i / kKT
-            // (granule 4*kk + grp): kbase + nt*8 pairs + 64*kk.
-            auto read_k = [&](int i) -> uint4 {
-                return *reinterpret_cast<const uint4 *>(kbase + 8 * (i % kKT) * kPairBytes + 64 * (i / kKT));
-            };
-            uint4 ka[kQkAhead];
-#pragma unroll
-            for (int i = 0; i < kQkAhead; ++i) ka[i] = read_k(i);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int i = 0; i < 8 * kKT; ++i) {
-#pragma unroll
-                for (int t = 0; t < NT; ++t)
-                    s[t][i % kKT] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(ka[i % kQkAhead]), as_h8(qb[t][i / kKT]),
-                                                                          s[t][i % kKT], 0, 0, 0);
-                if (i + kQkAhead < 8 * kKT) ka[i % kQkAhead] = read_k(i + kQkAhead);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            half8_t pb[NT][kKS];
-            float corr[NT];
-            bool rescale = false;
-            // A block wholly before the step's first new slot is visible to
-            // every row (wave-uniform test); otherwise mask key by key.  Rows
-            // past the unit's tokens are never written, so the open case
-            // needs no mask at all.
-            const bool open = key0 + kFold <= cu.ns;
-#pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                // Masked scores become -inf; the max is taken over the raw
-                // scores and scaled once (scale > 0 keeps the order and the
-                // rounding of the largest), and the probabilities below
-                // fold the scale into one fma.
-                if (!open) {  // wave-uniform: blocks of the cache prefix skip this
-#pragma unroll
-                    for (int nt = 0; nt < kKT; ++nt)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            bool vis;
-                            if constexpr (TREE) {
-                                // The cache before the step, then the new rows
-                                // in the node's bit set (bits only for the
-                                // step's nodes, so keys past the sequence drop
-                                // out).  Bitwise, so no lane branches.
-                                const int rel = key0 + 16 * nt + 4 * grp + i - cu.ns;
-                                const bool bit = ((qbits[t] >> (rel & 63)) & 1ull) != 0;
-                                vis = qvalid[t] & ((rel < 0) | ((rel < 64) & bit));
-                            } else {
-                                // key0 + 16nt + 4grp + i <= qslot (qslot < ctx)
-                                vis = qvalid[t] & (16 * nt + i <= qslot[t] - key0 - 4 * grp);
-                            }
-                            s[t][nt][i] = vis ? s[t][nt][i] : -INFINITY;
-                        }
-                }
-                float mx = -INFINITY;
+                // S^T for keys key0 + 16*nt + 4*grp + i, row `col` of each tile.
+                float4_t s[NT][kKT];
 #pragma unroll
                 for (int nt = 0; nt < kKT; ++nt)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[t][nt][i]);
-                mx = group4_max(mx) * scale;
-                // Move the reference max only on a jump past the slack (or
-                // from -inf, where acc and l are still zero).
-                const bool jump = mx > m[t] + kRescaleSlack;
-                const float mn = jump ? mx : m[t];
-                const float mu = (mn == -INFINITY) ? 0.0f : mn;  // rows with nothing visible yet
-                corr[t] = __builtin_amdgcn_exp2f(m[t] - mu);
-                rescale = rescale || (jump && m[t] != -INFINITY);
-                uint32_t pk[2 * kKT];
+                    for (int t = 0; t < NT; ++t) s[t][nt] = float4_t{0.f, 0.f, 0.f, 0.f};
+                // Operand i: key tile i % kKT (key 16*nt + col), k-step i / kKT
+                // (granule 4*kk + grp): kbase + nt*8 pairs + 64*kk.
+                auto read_k = [&](int i) -> uint4 {
+                    return *reinterpret_cast<const uint4 *>(kbase + 8 * (i % kKT) * kPairBytes + 64 * (i / kKT));
+                };
+                uint4 ka[kQkAhead];
 #pragma unroll
-                for (int nt = 0; nt < kKT; ++nt) {
-                    pk[2 * nt] = pack_p2(__builtin_amdgcn_exp2f(fmaf(s[t][nt][0], scale, -mu)),
-                                         __builtin_amdgcn_exp2f(fmaf(s[t][nt][1], scale, -mu)));
-                    pk[2 * nt + 1] = pack_p2(__builtin_amdgcn_exp2f(fmaf(s[t][nt][2], scale, -mu)),
-                                             __builtin_amdgcn_exp2f(fmaf(s[t][nt][3], scale, -mu)));
-                }
-                // l sums the fp16 probabilities PV uses.
-                constexpr uint32_t kOnes = 0x3c003c00u;  // fp16 pair (1, 1)
-                float psum = 0.0f;
-#pragma unroll
-                for (int i = 0; i < 2 * kKT; ++i) psum = dot2(pk[i], kOnes, psum);
-                l[t] = l[t] * corr[t] + psum;
-                m[t] = mn;
-#pragma unroll
-                for (int ks = 0; ks < kKS; ++ks)
-                    pb[t][ks] = __builtin_bit_cast(half8_t, make_uint4(pk[4 * ks], pk[4 * ks + 1], pk[4 * ks + 2],
-                                                                      pk[4 * ks + 3]));
-            }
-            // Rescale only when some row's reference max moved (wave-uniform).
-            if (__builtin_amdgcn_ballot_w64(rescale)) {
-#pragma unroll
-                for (int t = 0; t < NT; ++t)
-#pragma unroll
-                    for (int dt = 0; dt < 16; ++dt) acc[t][dt] *= corr[t];
-            }
-            // V^T operand of dim tile dt: ds_read_b64_tr_b16 gives lane c of
-            // a 16-lane group column c of the 4 x 16 block whose row r the
-            // group's lanes 4r..4r+3 address, 8 bytes each: here key
-            // 4*grp + r (then 16 + 4*grp + r), dims 16*dt + 4*(lane%4) ...
-            // Key 16*hh + 4*grp + vr, granule 2*dt + vs/2: for odd keys the
-            // swap of fours moves dims 32*dt.. by +-64 B, + when bit 1 of dt
-            // is clear, - when set, so two bases cover every dt.
-            const int vr = (lane & 15) >> 2;
-            const int vs = lane & 3;
-            const uint8_t *vb = kt + kTileBytes + key_off(4 * grp + vr) + 16 * (vs >> 1) + 8 * (vs & 1);
-            const uint8_t *vbase[2] = {vb + 64 * (vr & 1), vb - 64 * (vr & 1)};
-            // Operand i: dim tile i / kKS, keys 32*(i % kKS) .. (16 pairs on).
-            auto read_v = [&](int i) -> half8_t {
-                short4_t part[2];
-#pragma unroll
-                for (int hh = 0; hh < 2; ++hh) {
-                    const uint8_t *src =
-                        vbase[(i / kKS >> 1) & 1] + (16 * (i % kKS) + 8 * hh) * kPairBytes + 32 * (i / kKS);
-                    part[hh] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t *)src);
-                }
-                const uint2 v0 = __builtin_bit_cast(uint2, part[0]);
-                const uint2 v1 = __builtin_bit_cast(uint2, part[1]);
-                return __builtin_bit_cast(half8_t, make_uint4(v0.x, v0.y, v1.x, v1.y));
-            };
-            half8_t va[kPvAhead];
-#pragma unroll
-            for (int i = 0; i < kPvAhead; ++i) va[i] = read_v(i);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int i = 0; i < 16 * kKS; ++i) {
-#pragma unroll
-                for (int t = 0; t < NT; ++t)
-                    acc[t][i / kKS] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va[i % kPvAhead], pb[t][i % kKS],
-                                                                            acc[t][i / kKS], 0, 0, 0);
-                if (i + kPvAhead < 16 * kKS) va[i % kPvAhead] = read_v(i + kPvAhead);
+                for (int i = 0; i < kQkAhead; ++i) ka[i] = read_k(i);
                 __builtin_amdgcn_sched_barrier(0);
-            }
+#pragma unroll
+                for (int i = 0; i < 8 * kKT; ++i) {
+#pragma unroll
+                    for (int t = 0; t < NT; ++t)
+                        s[t][i % kKT] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(ka[i % kQkAhead]), as_h8(qb[t][i / kKT]),
+                                                                              s[t][i % kKT], 0, 0, 0);
+                    if (i + kQkAhead < 8 * kKT) ka[i % kQkAhead] = read_k(i + kQkAhead);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                half8_t pb[NT][kKS];
+                float corr[NT];
+                bool rescale = false;
+                // A block wholly before the step's first new slot is visible to
+                // every row (wave-uniform test); otherwise mask key by key.  Rows
+                // past the unit's tokens are never written, so the open case
+                // needs no mask at all.
+                const bool open = key0 + kFold <= cu.ns;
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    // Masked scores become -inf; the max is taken over the raw
+                    // scores and scaled once (scale > 0 keeps the order and the
+                    // rounding of the largest), and the probabilities below
+                    // fold the scale into one fma.
+                    if (!open) {  // wave-uniform: blocks of the cache prefix skip this
+#pragma unroll
+                        for (int nt = 0; nt < kKT; ++nt)
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                bool vis;
+                                if constexpr (TREE) {
+                                    // The cache before the step, then the new rows
+                                    // in the node's bit set (bits only for the
+                                    // step's nodes, so keys past the sequence drop
+                                    // out).  Bitwise, so no lane branches.
+                                    const int rel = key0 + 16 * nt + 4 * grp + i - cu.ns;
+                                    const bool bit = ((qbits[t] >> (rel & 63)) & 1ull) != 0;
+                                    vis = qvalid[t] & ((rel < 0) | ((rel < 64) & bit));
+                                } else {
+                                    // key0 + 16nt + 4grp + i <= qslot (qslot < ctx)
+                                    vis = qvalid[t] & (16 * nt + i <= qslot[t] - key0 - 4 * grp);
+                                }
+                                s[t][nt][i] = vis ? s[t][nt][i] : -INFINITY;
+                            }
+                    }
+                    float mx = -INFINITY;
+#pragma unroll
+                    for (int nt = 0; nt < kKT; ++nt)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[t][nt][i]);
+                    mx = group4_max(mx) * scale;
+                    // Move the reference max only on a jump past the slack (or
+                    // from -inf, where acc and l are still zero).
+                    const bool jump = mx > m[t] + kRescaleSlack;
+                    const float mn = jump ? mx : m[t];
+                    const float mu = (mn == -INFINITY) ? 0.0f : mn;  // rows with nothing visible yet
+                    corr[t] = __builtin_amdgcn_exp2f(m[t] - mu);
+                    rescale = rescale || (jump && m[t] != -INFINITY);
+                    uint32_t pk[2 * kKT];
+#pragma unroll
+                    for (int nt = 0; nt < kKT; ++nt) {
+                        pk[2 * nt] = pack_p2(__builtin_amdgcn_exp2f(fmaf(s[t][nt][0], scale, -mu)),
+                                             __builtin_amdgcn_exp2f(fmaf(s[t][nt][1], scale, -mu)));
+                        pk[2 * nt + 1] = pack_p2(__builtin_amdgcn_exp2f(fmaf(s[t][nt][2], scale, -mu)),
+                                                 __builtin_amdgcn_exp2f(fmaf(s[t][nt][3], scale, -mu)));
+                    }
+                    // l sums the fp16 probabilities PV uses.
+                    constexpr uint32_t kOnes = 0x3c003c00u;  // fp16 pair (1, 1)
+                    float psum = 0.0f;
+#pragma unroll
+                    for (int i = 0; i < 2 * kKT; ++i) psum = dot2(pk[i], kOnes, psum);
+                    l[t] = l[t] * corr[t] + psum;
+                    m[t] = mn;
+#pragma unroll
+                    for (int ks = 0; ks < kKS; ++ks)
+                        pb[t][ks] = __builtin_bit_cast(half8_t, make_uint4(pk[4 * ks], pk[4 * ks + 1], pk[4 * ks + 2],
+                                                                          pk[4 * ks + 3]));
+                }
+                // Rescale only when some row's reference max moved (wave-uniform).
+                if (__builtin_amdgcn_ballot_w64(rescale)) {
+#pragma unroll
+                    for (int t = 0; t < NT; ++t)
+#pragma unroll
+                        for (int dt = 0; dt < 16; ++dt) acc[t][dt] *= corr[t];
+                }
+                // V^T operand of dim tile dt: ds_read_b64_tr_b16 gives lane c of
+                // a 16-lane group column c of the 4 x 16 block whose row r the
+                // group's lanes 4r..4r+3 address, 8 bytes each: here key
+                // 4*grp + r (then 16 + 4*grp + r), dims 16*dt + 4*(lane%4) ...
+                // Key 16*hh + 4*grp + vr, granule 2*dt + vs/2: for odd keys the
+                // swap of fours moves dims 32*dt.. by +-64 B, + when bit 1 of dt
+                // is clear, - when set, so two bases cover every dt.
+                const int vr = (lane & 15) >> 2;
+                const int vs = lane & 3;
+                const uint8_t *vb = kt + kTileBytes + key_off(4 * grp + vr) + 16 * (vs >> 1) + 8 * (vs & 1);
+                const uint8_t *vbase[2] = {vb + 64 * (vr & 1), vb - 64 * (vr & 1)};
+                // Operand i: dim tile i / kKS, keys 32*(i % kKS) .. (16 pairs on).
+                auto read_v = [&](int i) -> half8_t {
+                    short4_t part[2];
+#pragma unroll
+                    for (int hh = 0; hh < 2; ++hh) {
+                        const uint8_t *src =
+                            vbase[(i / kKS >> 1) & 1] + (16 * (i % kKS) + 8 * hh) * kPairBytes + 32 * (i / kKS);
+                        part[hh] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t *)src);
+                    }
+                    const uint2 v0 = __builtin_bit_cast(uint2, part[0]);
+                    const uint2 v1 = __builtin_bit_cast(uint2, part[1]);
+                    return __builtin_bit_cast(half8_t, make_uint4(v0.x, v0.y, v1.x, v1.y));
+                };
+                half8_t va[kPvAhead];
+#pragma unroll
+                for (int i = 0; i < kPvAhead; ++i) va[i] = read_v(i);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < 16 * kKS; ++i) {
+#pragma unroll
+                    for (int t = 0; t < NT; ++t)
+                        acc[t][i / kKS] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va[i % kPvAhead], pb[t][i % kKS],
+                                                                                acc[t][i / kKS], 0, 0, 0);
+                    if (i + kPvAhead < 16 * kKS) va[i % kPvAhead] = read_v(i + kPvAhead);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
             ++n_done;
         }
@@ -558,9 +557,10 @@ __global__ __launch_bounds__(64 * WAVES) void mq_kernel(MultiQueryArgs a) {
                     }
                     if (NT > 1) __builtin_amdgcn_sched_barrier(0);
                 }
-            } else {
+            } else if (qvalid[t]) {
                 // Slot 2w: the unit began at or before this share (its first
-                // segment); slot 2w+1: the share's last segment.
+                // segment); slot 2w+1: the share's last segment.  (Rows past
+                // the tile's tokens are not merged: 10 of a nine-node tree's 64.)
                 const int slot = 2 * w + (cu.ub <= q0 ? 0 : 1);
                 const size_t rowi = static_cast<size_t>(slot) * kMqSlotRows + rho;
                 float *ar = a.ws_acc + rowi * kHeadDim;
