@@ -729,7 +729,7 @@ __global__ __launch_bounds__(64 * G) void combine_kernel(DecodeArgs a) {
 // combine_wide_kernel (any number of pieces: one long sequence over every CU
 // has 256): a workgroup per (sequence, query head, quarter of the head's
 // dims).  A wave takes four pieces per load instruction, 16 lanes x 4 dims
-// each, and kDepth such loads before it uses any, so NW = 16 waves hold 256
+// each, and kDepth such loads before it uses any, so NW waves hold 16 NW
 // pieces in flight at once; lane groups merge by shuffles and waves through
 // LDS.  Latency bounds it: with the whole head in four waves of one
 // workgroup, 16 pieces a wave at a time, 256 pieces took 9.0 us.
@@ -1124,11 +1124,17 @@ hipError_t launch_g(const DecodeArgs &a, hipStream_t s) {
     hipLaunchKernelGGL(decode_mfma_kernel<G>, dim3(a.n_wg, a.num_kv_heads / hpw), dim3(64 * hpw), 0, s, a);
     if ((e = hipGetLastError()) != hipSuccess || (e = mark(a.ev_after, s)) != hipSuccess) return e;
     const int units = a.n_seqs * a.num_kv_heads;
-    // Sixteen waves per workgroup while all of them fit the chip at once.
+    // Sixteen waves hold 256 pieces in flight, where a CU has one workgroup at
+    // most (a second round of them costs more: three sequences of 85 pieces
+    // 6.9 us, 4.2 with eight waves; one of 256 pieces 5.0 and 5.0, two 4.4 and
+    // 4.6).  Eight hold 128, worth it from about 50 pieces a sequence (four
+    // sequences of 64: 4.5 us, 4.8 with four waves); four hold the rest.
     if (a.few_pieces)
         hipLaunchKernelGGL((combine_kernel<G>), dim3(units), dim3(64 * G), 0, s, a);
-    else if (units * G * 4 <= 512)
+    else if (units * G * 4 <= 256)
         hipLaunchKernelGGL((combine_wide_kernel<G, 16>), dim3(units, G, 4), dim3(64 * 16), 0, s, a);
+    else if (a.n_wg > 48 * a.n_seqs)
+        hipLaunchKernelGGL((combine_wide_kernel<G, 8>), dim3(units, G, 4), dim3(64 * 8), 0, s, a);
     else
         hipLaunchKernelGGL((combine_wide_kernel<G, 4>), dim3(units, G, 4), dim3(64 * 4), 0, s, a);
     return hipGetLastError();

@@ -562,7 +562,7 @@ __global__ __launch_bounds__(64 * WAVES) void mq_kernel(MultiQueryArgs a) {
                 // segment); slot 2w+1: the share's last segment.  (Rows past
                 // the tile's tokens are not merged: 10 of a nine-node tree's 64.)
                 const int slot = 2 * w + (cu.ub <= q0 ? 0 : 1);
-                const size_t rowi = static_cast<size_t>(slot) * kMqSlotRows + rho;
+                const size_t rowi = static_cast<size_t>(slot) * (16 * WAVES * NT) + rho;
                 float *ar = a.ws_acc + rowi * kHeadDim;
 #pragma unroll
                 for (int dt = 0; dt < 16; ++dt)
@@ -603,6 +603,7 @@ __global__ __launch_bounds__(64 * kMqCombineRows) void mq_combine_kernel(MultiQu
     const int w0 = ld_uniform(rec + 3);
     const int w1 = ld_uniform(rec + 4);
     const int slot0 = ld_uniform(rec + 5);
+    const int slot_rows = 16 * a.n_waves * a.n_t;
     const int G = a.num_heads / a.num_kv_heads;
     const int rho = __builtin_amdgcn_readfirstlane(kMqCombineRows * blockIdx.y + (threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
@@ -624,7 +625,7 @@ __global__ __launch_bounds__(64 * kMqCombineRows) void mq_combine_kernel(MultiQu
             const int ww = wb + i;
             if (ww <= w1) {
                 const int slot = ww == w0 ? slot0 : 2 * ww;
-                const size_t rowi = static_cast<size_t>(slot) * kMqSlotRows + rho;
+                const size_t rowi = static_cast<size_t>(slot) * slot_rows + rho;
                 ml[i] = *reinterpret_cast<const float2 *>(a.ws_ml + rowi * 2);
                 v[i] = reinterpret_cast<const float4_t *>(a.ws_acc + rowi * kHeadDim)[lane];
             } else {

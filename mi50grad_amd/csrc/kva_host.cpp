@@ -80,9 +80,10 @@ struct kva_cache {
     float *d_ws_acc = nullptr;
     float *d_ws_ml = nullptr;
     uint64_t *d_timeline = nullptr;  // decode timeline records (kva_timeline_enable)
-    float *d_mq_acc = nullptr;  // multi-query partial slots [2*mq_max_wg][8][16][256]
+    float *d_mq_acc = nullptr;  // multi-query partial slots [2*mq_max_wg][128 or 256 rows][256]
     float *d_mq_ml = nullptr;
     int32_t mq_max_wg = 0;
+    bool mq_two_tiles = false;  // a step may take two row tiles per wave (256-row slots)
     float *d_proj = nullptr;    // projection partials [splits][tokens][rows]
     size_t part_floats = 0;     // what it holds
     size_t proj_floats = 0;     // the partials that kva_out_project's refusals are counted in
@@ -298,6 +299,15 @@ int32_t choose_wg(const kva_cache *c, int64_t pages) {
     return static_cast<int32_t>(std::max<int64_t>(1, w));
 }
 
+// Whether any step of this cache can be long enough for two row tiles per
+// wave: every tile of the longest step at the longest sequence.
+bool may_take_two_tiles(const kva_cache *c) {
+    const int32_t q = kva::mq_tile_tokens(c->group, 8, 1);
+    const int64_t tiles = (static_cast<int64_t>(c->cfg.max_step_tokens) / q + c->cfg.max_seqs) * c->cfg.num_kv_heads;
+    const int64_t blocks = static_cast<int64_t>(c->cfg.max_blocks_per_seq) * kva::kBlockTokens / 64 + 1;
+    return kva::mq_two_tiles(tiles * blocks, c->mq_max_wg);
+}
+
 // While a graph is being recorded, a call on another stream would run now
 // instead of being recorded, and a call that fails leaves a hole in the
 // recording: both are refused or remembered, and kva_graph_capture_end
@@ -370,9 +380,13 @@ int kva_create(const kva_config *cfg, kva_cache **out) {
     // device (against a nominal MI355X CU count) before they are refused.
     c->proj_floats = static_cast<size_t>(kva::kProjMaxSplits) * kva::kProjTokens *
                      (2 * static_cast<size_t>(cfg->num_heads) + 2 * cfg->num_kv_heads) * kva::kHeadDim;
-    c->part_floats = kva::kProjPartFactor * c->proj_floats;
+    // More where steps are long enough for splits of more tokens to use it.
+    const size_t step_floats = c->proj_floats / (kva::kProjMaxSplits * kva::kProjTokens) * kva::kGemmMaxSplits *
+                               static_cast<size_t>(cfg->max_step_tokens);
+    c->part_floats = std::max(c->proj_floats, std::min(kva::kProjPartFactor * c->proj_floats, step_floats));
     c->n_cu = kHostOnlyCus;
     c->mq_max_wg = c->n_cu;  // the device's CU count below
+    c->mq_two_tiles = may_take_two_tiles(c);
     if (!c->host_only) {
         auto cleanup = [&](int code) {
             kva_destroy(c);
@@ -406,7 +420,8 @@ int kva_create(const kva_config *cfg, kva_cache **out) {
             return cleanup(hip_fail(e, "hipMalloc(workspace ml)"));
         // Multi-query partial slots: two per workgroup, one workgroup per CU.
         c->mq_max_wg = c->n_cu;
-        const size_t mq_rows = static_cast<size_t>(2) * c->mq_max_wg * kva::kMqSlotRows;
+        c->mq_two_tiles = may_take_two_tiles(c);
+        const size_t mq_rows = static_cast<size_t>(2) * c->mq_max_wg * (c->mq_two_tiles ? 256 : 128);
         if ((e = hipMalloc(&c->d_mq_acc, mq_rows * kva::kHeadDim * sizeof(float))) != hipSuccess)
             return cleanup(hip_fail(e, "hipMalloc(multi-query workspace)"));
         if ((e = hipMalloc(&c->d_mq_ml, mq_rows * 2 * sizeof(float))) != hipSuccess)
@@ -663,13 +678,14 @@ int kva_step_begin(kva_cache *c, int32_t n_seqs, const int32_t *seq_ids, const i
     const int32_t mq_waves = kva::mq_waves_for(group, run_max);
     // Blocks of the step in one-tile units, each tile's keys taken as its
     // sequence's mean.
+    const int32_t one_tile_q = kva::mq_tile_tokens(group, mq_waves, 1);
     int64_t one_tile_blocks = 0;
     for (int32_t b = 0; b < n_seqs; ++b) {
-        const int64_t tiles = (n_new[b] + kva::mq_tile_tokens(group, mq_waves, 1) - 1) / kva::mq_tile_tokens(group, mq_waves, 1);
+        const int64_t tiles = (n_new[b] + one_tile_q - 1) / one_tile_q;
         one_tile_blocks += tiles * c->cfg.num_kv_heads * ((c->len[seq_ids[b]] + n_new[b] / 2) / 64 + 1);
     }
     const int32_t mq_nt =
-        mq_waves == 8 && !tree_bits && kva::mq_two_tiles(one_tile_blocks, c->mq_max_wg) ? 2 : 1;
+        mq_waves == 8 && !tree_bits && c->mq_two_tiles && kva::mq_two_tiles(one_tile_blocks, c->mq_max_wg) ? 2 : 1;
     const int32_t mq_q = kva::mq_tile_tokens(group, mq_waves, mq_nt);
     int64_t n_units = 0;
     for (int32_t b = 0; b < n_seqs; ++b)

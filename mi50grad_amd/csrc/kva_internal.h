@@ -55,7 +55,7 @@ hipError_t launch_append(const AppendArgs &a, hipStream_t s);
 constexpr int kProjTokens = 64;     // tokens the workspace refusals are counted in
 constexpr int kProjMaxSplits = 4;   // hidden split among workgroups, at most (proj_lds_kernel)
 constexpr int kGemmMaxSplits = 8;   // the same of the GEMM forms
-constexpr int kProjPartFactor = 4;  // partial workspace over kProjMaxSplits x kProjTokens tokens of every row
+constexpr size_t kProjPartFactor = 4;  // partial workspace over kProjMaxSplits x kProjTokens tokens of every row, at most
 constexpr int kProjWaves = 8;       // waves per workgroup
 constexpr int kProjRowTiles = 7;    // 16-row weight tiles per workgroup
 constexpr int kProjHiddenQuantum = 512;  // hidden must be a multiple of this
@@ -269,8 +269,8 @@ struct MultiQueryArgs {
     int32_t n_waves;          // waves per workgroup (4 or 8)
     int32_t n_t;              // 16-row MFMA tiles per wave (1 or 2: mq_two_tiles)
     int32_t q_tile;           // new tokens per unit tile: mq_tile_tokens(G, n_waves, n_t)
-    float *ws_acc;            // [2*n_wg][kMqSlotRows][256] partial slots
-    float *ws_ml;             // [2*n_wg][kMqSlotRows][2]
+    float *ws_acc;            // [2*n_wg][16*n_waves*n_t][256] partial slots
+    float *ws_ml;             // [2*n_wg][16*n_waves*n_t][2]
     // Output gate (null = none), as in DecodeArgs: new token t's row of
     // query head hq at gate + t*gate_stride + hq*256.
     const uint16_t *gate;
@@ -294,7 +294,6 @@ constexpr int mq_keys_for(int waves, bool tree_plan) { return (waves == 8 && !tr
 // half the time, so half the cost would do) 4 as well.
 constexpr int kMqUnitCost = 4;
 constexpr int kMqMaxGroup = 8;    // largest GQA group of the multi-query kernel
-constexpr int kMqSlotRows = 256;  // query rows of a partial slot (waves x 16 x tiles at most)
 constexpr int kMqCutWords = 8;    // int32 words of a cut-unit record (6 used)
 // Workgroups of a multi-query launch over `blocks` positions: one per CU (the
 // cap), at least 128 keys' blocks each.  kva_step_begin (the cut-unit
