@@ -409,13 +409,14 @@ const GemmForm kForms[] = {
     {256, 128, 0.96f, false, true, true, nullptr, launch_gemm<Tile256x128, kEpiOut>, launch_gemm<Tile256x128, kEpiPart>},
     {192, 128, 0.76f, false, true, true, nullptr, launch_gemm<Tile192x128, kEpiOut>, launch_gemm<Tile192x128, kEpiPart>},
     {128, 128, 0.64f, false, true, true, nullptr, launch_gemm<Tile128x128, kEpiOut>, launch_gemm<Tile128x128, kEpiPart>},
-    {64, 128, 0.47f, false, true, true, nullptr, launch_gemm<Tile64x128, kEpiOut>, launch_gemm<Tile64x128, kEpiPart>},
+    {64, 128, 0.60f, false, true, true, nullptr, launch_gemm<Tile64x128, kEpiOut>, launch_gemm<Tile64x128, kEpiPart>},
 };
 
 // The tile and the split of hidden for T tokens: the least estimated time.
 // A round of tiles (one per CU) costs its chunks plus about 3 us to start
-// and end, and no less than the operands take to stream at 5 TB/s; a split
-// adds its partials, written and read back, and the finish launch.  The
+// and end, and no less than the operands take to stream at 5 TB/s shared by
+// all CUs (48 tokens of 6144 -> 5120 take 20.6 us over four splits, 160
+// workgroups, and 17.7 over six, 240); a split adds its partials, written and read back, and the finish launch.  The
 // estimate is within 15 % of the measured times it was fitted to (64 to 2048
 // tokens of 5120 -> 14336 and 6144 -> 5120, and their halves and quarters):
 // 2048 tokens of 6144 -> 5120 take 137 us in 128 x 320 tiles (one round of
@@ -444,7 +445,12 @@ GemmPlan gemm_plan(const ProjectArgs &a, bool heads, int n_cu, size_t part_float
             if (splits > 1 && part > static_cast<double>(part_floats)) break;
             const double rounds = static_cast<double>((static_cast<int64_t>(tiles * splits) + n_cu - 1) / n_cu);
             const double walk = rounds * ((nc + splits - 1) / splits) * f.chunk_us;
-            double us = 3.0 * rounds + (walk > stream_us ? walk : stream_us);
+            // A CU streams its share of the operands: fewer workgroups than
+            // CUs stretch that time.  A tenth of the lesser term is a
+            // tie-break (a smaller tile walks the same stream more lightly).
+            const double fill = tiles * splits < n_cu ? n_cu / (tiles * splits) : 1.0;
+            const double stream = stream_us * fill;
+            double us = 3.0 * rounds + (walk > stream ? walk + 0.1 * stream : stream + 0.1 * walk);
             if (splits > 1) us += 4.0 + 8.0 * part / 5.0e6;
             if (!best.form || us < best_us) {
                 best = GemmPlan{&f, splits};
