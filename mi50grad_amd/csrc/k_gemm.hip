@@ -20,9 +20,9 @@
 //   whole tiles would leave most of the 256 CUs idle.
 // The O-projection of 2048 tokens (6144 -> 5120) ran as 32 launch pairs of
 // the 64-token form, each reading all of W_o: 1023 us; as 256 tiles of
-// 128 x 320 in one launch: 137.  181 tokens: Q/K/V 133 -> 52 us (56 tiles of
+// 128 x 320 in one launch: 137.  181 tokens: Q/K/V 133 -> 53 us (56 tiles of
 // 256 x 256 before, 224 of 192 x 128 over two splits now), O-projection
-// 102 -> 27.
+// 102 -> 27.  2048 tokens' Q/K/V: 278 (gemm_pair_kernel).
 //
 // Main loop.  Eight waves in a WM x (8 / WM) grid, v_mfma_f32_16x16x32_f16
 // with W rows as A and tokens as B.  K goes in chunks of 64 through S LDS
@@ -45,6 +45,8 @@
 // Tile order.  Tiles are dealt out XCD by XCD (workgroup i runs on XCD
 // i % 8): each XCD takes a contiguous run, so a row tile's weights are read
 // by one XCD and reused from its L2 by the token tiles beside each other.
+#include <algorithm>
+
 #include "k_common.h"
 #include "k_normrope.h"
 #include "kva_internal.h"
@@ -113,29 +115,38 @@ __device__ __forceinline__ void g_issue(uint32_t stage, __amdgpu_buffer_rsrc_t r
 
 __device__ __forceinline__ half8_t g_h8(uint4 v) { return __builtin_bit_cast(half8_t, v); }
 
-template <class T, int EPI>
-__global__ __launch_bounds__(64 * kGWaves) void gemm_kernel(ProjectArgs a) {
-    constexpr int kTM = T::kTM, kTN = T::kTN;
-    __shared__ __attribute__((aligned(16))) uint8_t ring[T::S * T::kStage];
-    // Per token of a head tile: RoPE position, sequence, slot, page id.
-    __shared__ int32_t meta[EPI == kEpiHead ? 4 : 1][EPI == kEpiHead ? T::BM : 1];
+// How gemm_pair_kernel cuts its row tiles.
+struct GemmPair {
+    int tall, all;         // workgroups of tall tiles, and of both
+    int heads;             // row tiles of the first kind
+    int hi, lo;            // tall tiles of one row tile of the first kind, of the others
+    int rest_hi, rest_lo;  // the same of the low ones
+};
 
+// A workgroup's LDS: the ring of stages, the facts of a head tile's tokens
+// (RoPE position, sequence, slot, page id) and the words of lines touched.
+template <class T, int EPI>
+struct GShared {
+    uint8_t ring[T::S * T::kStage];
+    int32_t meta[EPI == kEpiHead ? 4 : 1][EPI == kEpiHead ? T::BM : 1];
+    uint32_t touched[T::AHEAD > 0 ? kGWaves * 64 : 1];
+};
+
+// Workgroup i runs on XCD i % 8: deal each XCD a contiguous run of n tiles.
+__device__ __forceinline__ int g_deal(int i, int n) {
+    const int xcd = i & 7, q8 = n >> 3, r8 = n & 7;
+    return xcd * q8 + min(xcd, r8) + (i >> 3);
+}
+
+// One tile: token tile mt (first token t0 within the launch) of the n_mt that
+// a row tile has, row tile rt, and with kEpiPart slice `split` of `splits`.
+template <class T, int EPI>
+__device__ __forceinline__ void gemm_tile(const ProjectArgs &a, GShared<T, EPI> &sh, int t0, int mt, int n_mt, int rt,
+                                          int split, int splits) {
+    constexpr int kTM = T::kTM, kTN = T::kTN;
+    uint8_t *const ring = sh.ring;
+    auto &meta = sh.meta;
     const int N = a.n_a + a.n_b;
-    const int n_rt = (N + T::BN - 1) / T::BN;
-    const int n_mt = (a.n_tok + T::BM - 1) / T::BM;
-    const int splits = EPI == kEpiPart ? a.splits : 1;
-    const int n_tiles = n_rt * splits * n_mt;
-    // Workgroup i runs on XCD i % 8: deal each XCD a contiguous run of tiles.
-    const int xcd = blockIdx.x & 7, q8 = n_tiles >> 3, r8 = n_tiles & 7;
-    const int tau = xcd * q8 + min(xcd, r8) + static_cast<int>(blockIdx.x >> 3);
-    // Token tiles fastest, then row tiles, then splits, so that the tiles
-    // beside each other share a row tile's weights and a split's slice of x.
-    // (readfirstlane: quotients are computed in vector registers, and the
-    // loads' resources must be scalar.)
-    const int ws = __builtin_amdgcn_readfirstlane(tau / n_mt);
-    const int t0 = (tau - ws * n_mt) * T::BM;      // first token of the tile within the launch
-    const int split = EPI == kEpiPart ? __builtin_amdgcn_readfirstlane(ws / n_rt) : 0;
-    const int rt = ws - split * n_rt;
     const int n0 = rt * T::BN;                     // first stacked weight row
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
@@ -180,12 +191,11 @@ __global__ __launch_bounds__(64 * kGWaves) void gemm_kernel(ProjectArgs a) {
     // their operands (W: the token tiles of a row tile; X: the row tiles
     // beside it), so each touches its part of the rows of chunk c + AHEAD
     // and the loads themselves find all of them in L2.
-    __shared__ uint32_t touched[T::AHEAD > 0 ? kGWaves * 64 : 1];
-    const uint32_t touch0 = lds_addr(touched) + 256 * wv;
+    const uint32_t touch0 = lds_addr(sh.touched) + 256 * wv;
     uint32_t toff_w = 0x80000000u, toff_x = 0x80000000u;  // out of range: no access
     if constexpr (T::AHEAD > 0) {
         const int share_w = min(n_mt, kGXcdCus), share_x = max(1, kGXcdCus / n_mt);
-        const int row_w = (64 * wv + lane) * share_w + t0 / T::BM % share_w;
+        const int row_w = (64 * wv + lane) * share_w + mt % share_w;
         const int row_x = (64 * wv + lane) * share_x + rt % share_x;
         if (share_w > 1 && row_w < T::BN) toff_w = row_w * row_bytes;
         if (share_x > 1 && row_x < T::BM) toff_x = row_x * row_bytes;
@@ -373,7 +383,56 @@ __global__ __launch_bounds__(64 * kGWaves) void gemm_kernel(ProjectArgs a) {
     }
 }
 
+template <class T, int EPI>
+__global__ __launch_bounds__(64 * kGWaves) void gemm_kernel(ProjectArgs a) {
+    __shared__ __attribute__((aligned(16))) GShared<T, EPI> sh;
+    const int n_rt = (a.n_a + a.n_b + T::BN - 1) / T::BN;
+    const int n_mt = (a.n_tok + T::BM - 1) / T::BM;
+    const int splits = EPI == kEpiPart ? a.splits : 1;
+    const int tau = g_deal(blockIdx.x, n_rt * splits * n_mt);
+    // Token tiles fastest, then row tiles, then splits, so that the tiles
+    // beside each other share a row tile's weights and a split's slice of x.
+    // (readfirstlane: quotients are computed in vector registers, and the
+    // loads' resources must be scalar.)
+    const int ws = __builtin_amdgcn_readfirstlane(tau / n_mt);
+    const int mt = tau - ws * n_mt;
+    const int split = EPI == kEpiPart ? __builtin_amdgcn_readfirstlane(ws / n_rt) : 0;
+    gemm_tile<T, EPI>(a, sh, mt * T::BM, mt, n_mt, ws - split * n_rt, split, splits);
+}
+
+// Head tiles of two heights in one launch: tiles of TA's tokens for whole
+// rounds of the chip, then tiles of TB's for the rest.  Tiles of one height
+// leave the last round part empty: 2048 tokens of 5120 -> 14336 are 448 tiles
+// of 256 x 256, 1.75 rounds of 256 CUs, 298 us; 256 of those and 256 of
+// 192 x 256 take 278.  1300 tokens 268 -> 224 (192 and 128 against 616 tiles
+// of 128), 4000 618 -> 523.  Row tile r has k token
+// tiles of TA, k = p.hi for the first p.heads rows and p.lo after
+// them, and as many of TB as its other tokens need.
+template <class TA, class TB>
+__global__ __launch_bounds__(64 * kGWaves) void gemm_pair_kernel(ProjectArgs a, GemmPair p) {
+    static_assert(TA::BN == kHeadDim && TB::BN == kHeadDim, "head tiles");
+    __shared__ __attribute__((aligned(16))) union {
+        GShared<TA, kEpiHead> a;
+        GShared<TB, kEpiHead> b;
+    } sh;
+    const int i = blockIdx.x;
+    const bool tall = i < p.tall;
+    const int tau = tall ? g_deal(i, p.tall) : g_deal(i - p.tall, p.all - p.tall);
+    const int hi = tall ? p.hi : p.rest_hi, lo = tall ? p.lo : p.rest_lo;  // tiles of a row tile
+    const bool first = tau < p.heads * hi;
+    const int rel = first ? tau : tau - p.heads * hi;
+    const int per = max(1, first ? hi : lo);
+    const int row = __builtin_amdgcn_readfirstlane(rel / per);
+    const int mt = rel - row * per;
+    const int rt = first ? row : p.heads + row;
+    if (tall)
+        gemm_tile<TA, kEpiHead>(a, sh.a, mt * TA::BM, mt, per, rt, 0, 1);
+    else
+        gemm_tile<TB, kEpiHead>(a, sh.b, (first ? p.hi : p.lo) * TA::BM + mt * TB::BM, mt, per, rt, 0, 1);
+}
+
 using Tile256x256 = GTile<256, 256, 2, 2, 0>;
+using Tile192x256 = GTile<192, 256, 2, 2, 0>;
 using Tile128x256 = GTile<128, 256, 2, 3, 1>;
 using Tile64x256 = GTile<64, 256, 1, 3, 1>;
 using Tile128x320 = GTile<128, 320, 2, 2, 1>;
@@ -390,6 +449,12 @@ hipError_t launch_gemm(const ProjectArgs &a, hipStream_t s) {
     return hipGetLastError();
 }
 
+template <class TA, class TB>
+hipError_t launch_pair(const ProjectArgs &a, const GemmPair &p, hipStream_t s) {
+    hipLaunchKernelGGL((gemm_pair_kernel<TA, TB>), dim3(p.all), dim3(64 * kGWaves), 0, s, a, p);
+    return hipGetLastError();
+}
+
 // The tile shapes, and what a 64-wide k chunk of each takes on a full chip
 // (us, measured at hidden 5120 and 6144).
 struct GemmForm {
@@ -402,15 +467,50 @@ struct GemmForm {
 };
 const GemmForm kForms[] = {
     {256, 256, 1.88f, true, false, false, launch_gemm<Tile256x256, kEpiHead>, nullptr, nullptr},
+    {192, 256, 1.50f, true, false, false, launch_gemm<Tile192x256, kEpiHead>, nullptr, nullptr},
     {128, 256, 1.05f, true, true, true, launch_gemm<Tile128x256, kEpiHead>, launch_gemm<Tile128x256, kEpiOut>,
      launch_gemm<Tile128x256, kEpiPart>},
     {64, 256, 0.84f, true, false, true, launch_gemm<Tile64x256, kEpiHead>, nullptr, launch_gemm<Tile64x256, kEpiPart>},
     {128, 320, 1.30f, false, true, false, nullptr, launch_gemm<Tile128x320, kEpiOut>, nullptr},
-    {256, 128, 0.96f, false, true, true, nullptr, launch_gemm<Tile256x128, kEpiOut>, launch_gemm<Tile256x128, kEpiPart>},
-    {192, 128, 0.76f, false, true, true, nullptr, launch_gemm<Tile192x128, kEpiOut>, launch_gemm<Tile192x128, kEpiPart>},
-    {128, 128, 0.64f, false, true, true, nullptr, launch_gemm<Tile128x128, kEpiOut>, launch_gemm<Tile128x128, kEpiPart>},
+    {256, 128, 0.96f, false, true, true, nullptr, launch_gemm<Tile256x128, kEpiOut>,
+     launch_gemm<Tile256x128, kEpiPart>},
+    {192, 128, 0.76f, false, true, true, nullptr, launch_gemm<Tile192x128, kEpiOut>,
+     launch_gemm<Tile192x128, kEpiPart>},
+    {128, 128, 0.64f, false, true, true, nullptr, launch_gemm<Tile128x128, kEpiOut>,
+     launch_gemm<Tile128x128, kEpiPart>},
     {64, 128, 0.60f, false, true, true, nullptr, launch_gemm<Tile64x128, kEpiOut>, launch_gemm<Tile64x128, kEpiPart>},
 };
+
+// The heights that gemm_pair_kernel is built for: indices into kForms.
+struct GemmPairForm {
+    int tall, low;
+    hipError_t (*launch)(const ProjectArgs &, const GemmPair &, hipStream_t);
+};
+const GemmPairForm kPairs[] = {
+    {0, 1, launch_pair<Tile256x256, Tile192x256>},
+    {0, 2, launch_pair<Tile256x256, Tile128x256>},
+    {1, 2, launch_pair<Tile192x256, Tile128x256>},
+};
+
+// Tall tiles for whole rounds of the chip, shared out over n_rt row
+// tiles as evenly as leaves the fewest low ones (room: workgroups of those rounds).
+GemmPair pair_tiles(int T, int n_rt, int bm, int bm_low, int64_t room) {
+    GemmPair best{0, 0, 0, 0, 0, 0, 0};
+    const int most = T / bm;
+    for (int lo = 0; lo <= most; ++lo) {
+        if (static_cast<int64_t>(n_rt) * lo > room) break;
+        for (int hi = lo + 1; hi <= most; ++hi) {
+            const int64_t more = (room - static_cast<int64_t>(n_rt) * lo) / (hi - lo);
+            const int heads = static_cast<int>(std::min<int64_t>(n_rt, more));
+            const int rest_hi = (T - hi * bm + bm_low - 1) / bm_low, rest_lo = (T - lo * bm + bm_low - 1) / bm_low;
+            const int tall = heads * hi + (n_rt - heads) * lo;
+            const int all = tall + heads * rest_hi + (n_rt - heads) * rest_lo;
+            if (tall > 0 && (best.all == 0 || all - tall < best.all - best.tall))
+                best = GemmPair{tall, all, heads, hi, lo, rest_hi, rest_lo};
+        }
+    }
+    return best;
+}
 
 // The tile and the split of hidden for T tokens: the least estimated time.
 // A round of tiles (one per CU) costs its chunks plus about 3 us to start
@@ -427,12 +527,14 @@ const GemmForm kForms[] = {
 struct GemmPlan {
     const GemmForm *form;
     int splits;
+    const GemmPairForm *pair;  // two heights instead of form
+    GemmPair cut;
 };
 GemmPlan gemm_plan(const ProjectArgs &a, bool heads, int n_cu, size_t part_floats) {
     const int T = a.n_tok, N = a.n_a + a.n_b;
     const int nc = a.hidden / kGKc;
     const double stream_us = 2.0 * a.hidden * (static_cast<double>(N) + T) / 5.0e6;
-    GemmPlan best{nullptr, 1};
+    GemmPlan best{};
     double best_us = 0;
     for (const GemmForm &f : kForms) {
         // Row offsets within a tile are 32-bit.
@@ -453,7 +555,26 @@ GemmPlan gemm_plan(const ProjectArgs &a, bool heads, int n_cu, size_t part_float
             double us = 3.0 * rounds + (walk > stream ? walk + 0.1 * stream : stream + 0.1 * walk);
             if (splits > 1) us += 4.0 + 8.0 * part / 5.0e6;
             if (!best.form || us < best_us) {
-                best = GemmPlan{&f, splits};
+                best.form = &f;
+                best.splits = splits;
+                best_us = us;
+            }
+        }
+    }
+    // Two heights, where one leaves its last round part empty.
+    for (const GemmPairForm &f : kPairs) {
+        const GemmForm &ft = kForms[f.tall], &fl = kForms[f.low];
+        if (!heads || !best.form || best.splits > 1 || a.n_a % ft.bn != 0) break;
+        const int n_rt = N / ft.bn;
+        for (int r = 1; static_cast<int64_t>(r) * n_cu * ft.bm < static_cast<int64_t>(T) * n_rt; ++r) {
+            const GemmPair cut = pair_tiles(T, n_rt, ft.bm, fl.bm, static_cast<int64_t>(r) * n_cu);
+            if (cut.all <= cut.tall) continue;
+            const int more = (cut.all - cut.tall + n_cu - 1) / n_cu;
+            const double walk = nc * (r * ft.chunk_us + more * fl.chunk_us);
+            const double us = 3.0 * (r + more) + (walk > stream_us ? walk + 0.1 * stream_us : stream_us + 0.1 * walk);
+            if (us < best_us) {
+                best.pair = &f;
+                best.cut = cut;
                 best_us = us;
             }
         }
@@ -469,6 +590,7 @@ hipError_t launch_gemm_project(ProjectArgs &a, bool heads, int n_cu, size_t part
     const GemmPlan plan = gemm_plan(a, heads, n_cu, part_floats);
     if (!plan.form) return hipErrorInvalidValue;
     a.splits = plan.splits;
+    if (plan.pair) return plan.pair->launch(a, plan.cut, s);
     if (a.splits > 1) return plan.form->launch_part(a, s);
     return (heads ? plan.form->launch_head : plan.form->launch_out)(a, s);
 }
