@@ -375,7 +375,7 @@ int kva_create(const kva_config *cfg, kva_cache **out) {
                                          sizeof(int32_t)),
                             256);
     c->stage_bytes = std::max(c->step_bytes, c->aux_bytes);
-    // Projection partials: every split of one launch pair's tokens.  Sized
+    // Projection partials: every split of kProjTokens tokens.  Sized
     // for host-only caches too, whose calls are validated exactly as on the
     // device (against a nominal MI355X CU count) before they are refused.
     c->proj_floats = static_cast<size_t>(kva::kProjMaxSplits) * kva::kProjTokens *
@@ -1307,7 +1307,7 @@ static int out_project_impl(kva_cache *c, const void *attn, int32_t n_tok, int32
     a.n_b = 0;
     a.hidden = q_dim;
     a.splits = project_splits(c, q_dim, n_out);
-    // One launch pair's partials: [splits][its tokens][n_out] floats.
+    // What is refused: [splits][up to kProjTokens tokens][n_out] floats.
     const int64_t chunk_tok = std::min(n_tok, kva::kProjTokens);
     if (static_cast<size_t>(a.splits) * chunk_tok * n_out > c->proj_floats)
         return fail(KVA_ERR_INVALID_ARG, "n_out %d x %lld tokens exceeds the projection workspace (%zu floats)", n_out,
@@ -1316,11 +1316,14 @@ static int out_project_impl(kva_cache *c, const void *attn, int32_t n_tok, int32
     a.part = c->d_proj;
     a.ev_before = c->kev_before;
     a.ev_after = c->kev_after;
-    a.y_out = static_cast<uint16_t *>(out);
-    a.residual = static_cast<const uint16_t *>(residual);
-    a.x = static_cast<const uint16_t *>(attn);
-    a.n_tok = n_tok;
-    KVA_HIP(kva::launch_out_project(a, c->n_cu, c->part_floats, static_cast<hipStream_t>(stream)));
+    for (int32_t t0 = 0; t0 < n_tok; t0 += kva::kBigProjMaxTokens) {
+        const size_t at0 = static_cast<size_t>(t0) * n_out;
+        a.x = static_cast<const uint16_t *>(attn) + static_cast<size_t>(t0) * q_dim;
+        a.y_out = static_cast<uint16_t *>(out) + at0;
+        a.residual = residual ? static_cast<const uint16_t *>(residual) + at0 : nullptr;
+        a.n_tok = std::min(kva::kBigProjMaxTokens, n_tok - t0);
+        KVA_HIP(kva::launch_out_project(a, c->n_cu, c->part_floats, static_cast<hipStream_t>(stream)));
+    }
     return KVA_OK;
 }
 

@@ -99,7 +99,7 @@ struct ProjectArgs {
     // fp16(x W_o^T + residual), both [T][n_a]; residual nullable, may be y_out.
     uint16_t *y_out;
     const uint16_t *residual;
-    // Events around the GEMM kernel of a launch pair (null: none), as in
+    // Events around the product's launch (null: none), as in
     // DecodeArgs.
     hipEvent_t ev_before, ev_after;
 };

@@ -188,9 +188,9 @@ class PagedKVCache:
                   table_rows, _ptr(q_out), _ptr(q_gate_out), _ptr(kv_out), stream)
 
     def project_path(self) -> str:
-        """Which path the last project_append took: "kernels" (the split-K
-        projection kernels, 64 tokens per launch pair) or "prefill_gemm" (one
-        GEMM launch over every token, the epilogue fused)."""
+        """Which path the last project_append took: "kernels" (steps of up to
+        64 tokens) or "prefill_gemm" (larger ones: one launch of GEMM tiles,
+        and a finish launch where hidden is split)."""
         p = ctypes.c_int32()
         _lib.call("kva_get_project_path", self.handle, ctypes.byref(p))
         return {0: "kernels", 1: "prefill_gemm"}[p.value]

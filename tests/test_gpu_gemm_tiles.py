@@ -54,13 +54,14 @@ def test_project_tiles_exact(device, hidden, n_new):
 
 
 # Head tiles of two heights in one launch: 192 then 128 tokens (1200), 256
-# then 192 (2048, and 1990 with a ragged last tile), and one height of 192.
-@pytest.mark.parametrize("n_new", [[1200], [2048], [1000, 990], [700]])
+# then 192 (2048, and 1990 with a ragged last tile), one height of 192, and
+# rows of more tiles than the plan's search spans (21 tall ones at 4090).
+@pytest.mark.parametrize("n_new", [[1200], [2048], [1000, 990], [700], [4090]])
 def test_project_two_heights_exact(device, n_new):
     rng = np.random.default_rng(sum(n_new))
     lengths = [int(x) for x in rng.integers(0, 60, len(n_new))]
     say(f"project_append two heights n_new {n_new}")
-    tables = Tables(device, 2304)
+    tables = Tables(device, sum(n_new) + 256)
     cache, kr, vr, exp, got, _, _, _, _ = _run(device, rng, lengths, n_new, 512, True, tables)
     q, gate, k_raw, k, v = exp
     assert np.array_equal(_bits(got["kv"][:, 0]), _bits(k_raw))
