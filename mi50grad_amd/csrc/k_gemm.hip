@@ -91,8 +91,8 @@ struct GTile {
 // at one logical granule must land on distinct 16-byte bank groups whether
 // the LDS serves 8 lanes per 128-byte cycle or 16 per 256-byte cycle: two
 // 128-byte rows share a 256-byte cycle, so the even rows take granules 0..7
-// and the odd rows the same set XORed by 4.  The counters read zero bank
-// conflicts.
+// and the odd rows the same set XORed by 4.  The main loop has no bank
+// conflicts (the head epilogue's are 0.3 % of a launch of 2048 tokens).
 __device__ __forceinline__ int g_swizzle(int r) { return ((r >> 1) ^ ((r & 1) << 2)) & 7; }
 
 // LDS byte offset of row r's 16-byte granule g within a stage's X or W part.
