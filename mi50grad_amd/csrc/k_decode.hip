@@ -34,6 +34,8 @@
 //   PV: lane owns dims 4*lane..4*lane+3 of all G heads; tokens t and t+4
 //       are paired so one v_dot2_f32_f16 folds two tokens; the pair's
 //       probabilities (row t's) reach every lane by an LDS broadcast.
+#include <type_traits>
+
 #include "k_common.h"
 #include "k_normrope.h"
 #include "kva_internal.h"
@@ -826,10 +828,24 @@ __global__ __launch_bounds__(64 * NW) void combine_wide_kernel(DecodeArgs a) {
     store(at, lt);
 }
 
+// Query heads a workgroup from which whole_kernel walks pages: where the
+// vector unit's share of a half page, which grows with the heads, passes its
+// loads'.  A layer of 40 ragged sequences (six heads a workgroup) of up to
+// 200, 450, 700 and 1000 rows takes 14.5, 19.3, 24.0 and 42.0 us on pages,
+// 16.4, 24.2, 30.5 and 45.4 on half pages; 64 of 450 rows 33.5 against 36.6,
+// with eight heads 35.5 against 37.5.  Three heads (32 sequences of 200, 450
+// and 1000 rows) lose, 14.7, 20.2 and 39.6 against 13.7, 18.5 and 35.2, and
+// two (16) too, 13.4, 18.6 and 30.6 against 11.6, 15.2 and 24.4: there a wave
+// waits for its loads, and half pages keep a third one in flight.
+constexpr int kWholePageHeads = 6;
+
 // Whole-sequence decode for steps of short sequences: a workgroup walks one
-// sequence for one kv head alone, its eight waves taking half pages w, w+8,
-// w+16, ... (8 token rows each, up to three in flight per wave); the waves
-// merge through LDS and write the output.  No partials and no combine
+// sequence for one kv head alone, its eight waves taking pieces w, w+8,
+// w+16, ...: half pages (8 token rows, up to three in flight per wave) with
+// both products on the vector unit, or, from kWholePageHeads query heads a
+// workgroup, pages with the scores on the matrix unit as in
+// decode_mfma_kernel (compute_page).  The waves merge through LDS and write
+// the output.  No partials and no combine
 // launch: a step of a few pages per sequence is bound by its launches, its
 // memory round trips and the VALU work of each CU, not by bandwidth.  The
 // G query heads of a kv head are split among a.whole workgroups of GP heads
@@ -848,9 +864,12 @@ __global__ __launch_bounds__(64 * NW) void combine_wide_kernel(DecodeArgs a) {
 // more partial (its score from the rounded K row, probability 1, its V row).
 template <int GP, bool kFused>
 __global__ __launch_bounds__(64 * kWholeWaves) void whole_kernel(DecodeArgs a) {
+    constexpr bool kPages = GP >= kWholePageHeads;
+    using Buffer = std::conditional_t<kPages, Page, HalfPage>;
+    constexpr int kRows = kPages ? kBlockTokens : kHalf;  // of a piece
     __shared__ uint4 q_lds[GP * 32];
     __shared__ uint4 kv_new[kFused ? 64 : 1];  // fused: the new K (normalised) and V rows
-    __shared__ uint32_t p_lds[kWholeWaves * 32];
+    __shared__ uint32_t p_lds[kWholeWaves * 64];
     __shared__ float4 mrg_acc[kWholeWaves * GP * 64];
     __shared__ float mrg_ml[(kWholeWaves + 1) * GP * 2];
     __shared__ uint64_t tl_t[2];  // timeline: entry and first-issue times
@@ -940,11 +959,11 @@ __global__ __launch_bounds__(64 * kWholeWaves) void whole_kernel(DecodeArgs a) {
                      ap.sin_tab + static_cast<size_t>(pos) * half_rot, half_rot, l32);
     }
 
-    const int n_hp = (max(walk, 0) + kHalf - 1) / kHalf;
-    const int n_i = wave < n_hp ? (n_hp - wave + kWholeWaves - 1) / kWholeWaves : 0;
-    const uint32_t koff = r * row_bytes + 16 * j;
+    const int n_pc = (max(walk, 0) + kRows - 1) / kRows;
+    const int n_i = wave < n_pc ? (n_pc - wave + kWholeWaves - 1) / kWholeWaves : 0;
+    const uint32_t koff = kPages ? j * row_bytes + 128 * r : r * row_bytes + 16 * j;
     const uint32_t voff = 8 * lane;
-    // Issue this wave's i-th half page into p (a no-op load past the list).
+    // Issue this wave's i-th piece into p (a no-op load past the list).
     // Block id of page pg (wave-uniform): the first 64 from the lanes' ids,
     // later ones from the table row by a vector load, which the compiler
     // keeps inside its branch (a scalar load it would issue for every page,
@@ -954,16 +973,21 @@ __global__ __launch_bounds__(64 * kWholeWaves) void whole_kernel(DecodeArgs a) {
         if (pg < 64) return __builtin_amdgcn_readlane(ids, pg);
         return __builtin_amdgcn_readfirstlane(row[pg]);
     };
-    auto issue = [&](HalfPage &p, int i) {
+    auto issue = [&](Buffer &p, int i) {
         const bool on = i < n_i;
-        const int hp = on ? wave + kWholeWaves * i : 0;
-        const int pg = hp >> 1;
-        const int id = page_of(pg);
-        const size_t ofs = static_cast<size_t>(id) * page_bytes + static_cast<size_t>(hp & 1) * kHalf * row_bytes;
-        load_half(p, kpool + ofs, vpool + ofs, min(kHalf, walk - hp * kHalf), on, koff, voff, row_bytes);
+        const int pc = on ? wave + kWholeWaves * i : 0;
+        const int id = page_of(kPages ? pc : pc >> 1);
+        const int lim = min(kRows, walk - pc * kRows);
+        if constexpr (kPages) {
+            const size_t ofs = static_cast<size_t>(id) * page_bytes;
+            load_page(p, kpool + ofs, vpool + ofs, lim, on, koff, voff, row_bytes);
+        } else {
+            const size_t ofs = static_cast<size_t>(id) * page_bytes + static_cast<size_t>(pc & 1) * kHalf * row_bytes;
+            load_half(p, kpool + ofs, vpool + ofs, lim, on, koff, voff, row_bytes);
+        }
     };
-    constexpr int kStages = GP <= 6 ? 3 : 2;
-    HalfPage A, B, C;
+    constexpr int kStages = !kPages && GP <= 6 ? 3 : 2;
+    Buffer A, B, C;
     issue(A, 0);
     if (kStages == 3) issue(B, 1);
     if (a.timeline && threadIdx.x == 0) tl_t[1] = __builtin_amdgcn_s_memrealtime();
@@ -992,22 +1016,31 @@ __global__ __launch_bounds__(64 * kWholeWaves) void whole_kernel(DecodeArgs a) {
         if (qi < GP * 32) q_lds[qi] = qin;
     }
     __syncthreads();
-    uint4 qv[GP][2];
+    // The query rows as MFMA columns (pages), or dims 8j.. and 128 + 8j.. of
+    // each (half pages).
+    uint4 qb[8], qv[GP][2];
+    if constexpr (kPages) {
 #pragma unroll
-    for (int g = 0; g < GP; ++g) {
-        qv[g][0] = q_lds[g * 32 + j];
-        qv[g][1] = q_lds[g * 32 + 16 + j];
+        for (int k = 0; k < 8; ++k) qb[k] = j < GP ? q_lds[j * 32 + 8 * r + k] : make_uint4(0, 0, 0, 0);
+    } else {
+#pragma unroll
+        for (int g = 0; g < GP; ++g) {
+            qv[g][0] = q_lds[g * 32 + j];
+            qv[g][1] = q_lds[g * 32 + 16 + j];
+        }
     }
 
-    WaveState<GP> st;
+    std::conditional_t<kPages, MfmaState<GP>, WaveState<GP>> st;
     reset(st);
-    int i = 0;  // the half page folded in next
-    auto step = [&](HalfPage &cr, HalfPage &nr) -> bool {
+    int i = 0;  // the piece folded in next
+    auto step = [&](Buffer &cr, Buffer &nr) -> bool {
         issue(nr, i + kStages - 1);
         __builtin_amdgcn_sched_barrier(0);
-        if (i < n_i) {
-            compute_half<GP>(st, cr, qv, r, j, min(kHalf, walk - (wave + kWholeWaves * i) * kHalf),
-                             p_lds + 32 * wave);
+        const int lim = min(kRows, walk - (wave + kWholeWaves * i) * kRows);
+        if constexpr (kPages) {
+            if (i < n_i) compute_page<GP>(st, cr, qb, lane, lim, p_lds + 64 * wave);
+        } else if (i < n_i) {
+            compute_half<GP>(st, cr, qv, r, j, lim, p_lds + 64 * wave);
         } else {
             consume(cr);
         }
@@ -1053,15 +1086,24 @@ __global__ __launch_bounds__(64 * kWholeWaves) void whole_kernel(DecodeArgs a) {
             }
         }
     }
+    if constexpr (kPages) {
+        const float lt = group4_sum(st.l);  // the four lane groups hold disjoint rows
+        if (lane < GP) {
+            mrg_ml[(wave * GP + lane) * 2] = st.m;
+            mrg_ml[(wave * GP + lane) * 2 + 1] = lt;
+        }
+    }
 #pragma unroll
     for (int g = 0; g < GP; ++g) {
-        float lt = st.l[g];  // the four rows hold disjoint tokens
-        lt += __shfl_xor(lt, 16);
-        lt += __shfl_xor(lt, 32);
         mrg_acc[(wave * GP + g) * 64 + lane] = make_float4(st.acc[g][0], st.acc[g][1], st.acc[g][2], st.acc[g][3]);
-        if (lane == 0) {
-            mrg_ml[(wave * GP + g) * 2] = st.m[g];
-            mrg_ml[(wave * GP + g) * 2 + 1] = lt;
+        if constexpr (!kPages) {
+            float lt = st.l[g];  // the four rows hold disjoint tokens
+            lt += __shfl_xor(lt, 16);
+            lt += __shfl_xor(lt, 32);
+            if (lane == 0) {
+                mrg_ml[(wave * GP + g) * 2] = st.m[g];
+                mrg_ml[(wave * GP + g) * 2 + 1] = lt;
+            }
         }
     }
     __syncthreads();
