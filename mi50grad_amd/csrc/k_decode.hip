@@ -17,8 +17,8 @@
 //       acc) per head for combine_kernel.
 //   whole_kernel: steps of short sequences (no combine): a workgroup walks
 //       one sequence for one kv head and a group of its query heads, eight
-//       waves on half pages with QK and PV on v_dot2_f32_f16 (below),
-//       merged through LDS; optionally with the step's append fused in.
+//       waves on half pages with QK and PV on v_dot2_f32_f16 (below), or
+//       with many heads on pages as above, merged through LDS; optionally with the step's append fused in.
 //
 // The whole-sequence form's half page, per wave (lane = 16*r + j):
 //   loads: a ring of register buffers; buffer loads through a per-page
@@ -986,7 +986,7 @@ __global__ __launch_bounds__(64 * kWholeWaves) void whole_kernel(DecodeArgs a) {
             load_half(p, kpool + ofs, vpool + ofs, lim, on, koff, voff, row_bytes);
         }
     };
-    constexpr int kStages = !kPages && GP <= 6 ? 3 : 2;
+    constexpr int kStages = kPages ? 2 : 3;
     Buffer A, B, C;
     issue(A, 0);
     if (kStages == 3) issue(B, 1);
@@ -1068,7 +1068,7 @@ __global__ __launch_bounds__(64 * kWholeWaves) void whole_kernel(DecodeArgs a) {
 
     // Merge the eight waves: each leaves (m, l, acc) in LDS; thread
     // (g, lane) merges head g's four dims 4*lane..4*lane+3.  A wave that had
-    // no half page left m = -inf, l = acc = 0 and weighs nothing.  Fused:
+    // no piece left m = -inf, l = acc = 0 and weighs nothing.  Fused:
     // wave g < GP adds head g's score of the new token as partial 8 (its V
     // row is read from LDS at the merge).
     const float qk_scale = kLog2e / 16.0f;
