@@ -181,7 +181,9 @@ int kva_append_qknorm_rope(kva_cache *cache, int32_t layer, void *q, void *k,
  * kva_decode / kva_prefill / kva_tree_verify); q_gate_out [T, num_heads,
  * 256] (Q_gate as projected, the gate of kva_decode_gated with gate_stride
  * num_heads*256; may be NULL); kv_out [T, 2, num_kv_heads, 256] (K and V as
- * projected, the reference's d_kv_fused; may be NULL).  16-byte aligned.   */
+ * projected, the reference's d_kv_fused; may be NULL).  16-byte aligned.
+ * q_out may be x itself where num_heads*256 <= hidden: an output that
+ * overlaps x or a weight goes through partials, which is slower.           */
 int kva_project_append(kva_cache *cache, int32_t layer, const void *x, int32_t hidden,
                        const void *w_q_fused, const void *w_kv_fused,
                        const void *q_norm_w, const void *k_norm_w,
@@ -197,6 +199,14 @@ int kva_project_append(kva_cache *cache, int32_t layer, const void *x, int32_t h
 #define KVA_PROJECT_KERNELS 0
 #define KVA_PROJECT_PREFILL_GEMM 1
 int kva_get_project_path(const kva_cache *cache, int32_t *path);
+/* The launch of the last kva_project_append or kva_out_project on this cache
+ * that passed its checks (its first, where it took several; on a host-only
+ * cache the one it would have made): tokens and weight rows of a GEMM tile
+ * (0: weights streamed past x held in registers), tokens of the low tiles of
+ * a launch of two heights (0: one height), slices that hidden was split
+ * into, and whether fp32 partials went to a finish kernel.                 */
+int kva_get_product_plan(const kva_cache *cache, int32_t *tile_tokens, int32_t *low_tokens,
+                         int32_t *tile_rows, int32_t *splits, int32_t *partial);
 /* Output projection of the (gated) attention rows, the consumer of
  * kva_decode_gated: out[t] = fp16(attn[t] . W_o^T + residual[t]) for
  * t < n_tok, accumulated in fp32 and rounded once after the residual add.
@@ -205,8 +215,9 @@ int kva_get_project_path(const kva_cache *cache, int32_t *path);
  * 2085, launcher engine.py:2434-2455, kernel gemv_fp16_v2.hip:22-87) for
  * all n_tok rows at once.  attn [n_tok, q_dim], w_o [n_out, q_dim] (row
  * major), residual and out [n_tok, n_out], fp16, 16-byte aligned; residual
- * may be NULL (no add) or equal to out (in place).  q_dim a multiple of 512,
- * n_out a multiple of 16 and at most (2*num_heads + 2*num_kv_heads)*256
+ * may be NULL (no add) or equal to out (in place); out may be attn itself
+ * where n_out <= q_dim (through partials, which is slower).  q_dim a multiple
+ * of 512, n_out a multiple of 16 and at most (2*num_heads + 2*num_kv_heads)*256
  * (the projection workspace).  Uses no step state.                        */
 int kva_out_project(kva_cache *cache, const void *attn, int32_t n_tok, int32_t q_dim,
                     const void *w_o, int32_t n_out, const void *residual, void *out,

@@ -46,6 +46,7 @@
 // i % 8): each XCD takes a contiguous run, so a row tile's weights are read
 // by one XCD and reused from its L2 by the token tiles beside each other.
 #include <algorithm>
+#include <iterator>
 
 #include "k_common.h"
 #include "k_normrope.h"
@@ -114,14 +115,6 @@ __device__ __forceinline__ void g_issue(uint32_t stage, __amdgpu_buffer_rsrc_t r
 }
 
 __device__ __forceinline__ half8_t g_h8(uint4 v) { return __builtin_bit_cast(half8_t, v); }
-
-// How gemm_pair_kernel cuts its row tiles.
-struct GemmPair {
-    int tall, all;         // workgroups of tall tiles, and of both
-    int heads;             // row tiles of the first kind
-    int hi, lo;            // tall tiles of one row tile of the first kind, of the others
-    int rest_hi, rest_lo;  // the same of the low ones
-};
 
 // A workgroup's LDS: the ring of stages, the facts of a head tile's tokens
 // (RoPE position, sequence, slot, page id) and the words of lines touched.
@@ -518,6 +511,8 @@ GemmPair pair_tiles(int T, int n_rt, int bm, int bm_low, int64_t room) {
     return best;
 }
 
+}  // namespace
+
 // The tile and the split of hidden for T tokens: the least estimated time.
 // A round of tiles (one per CU) costs its chunks plus about 3 us to start
 // and end, and no less than the operands take to stream at 5 TB/s shared by
@@ -529,28 +524,27 @@ GemmPair pair_tiles(int T, int n_rt, int bm, int bm_low, int64_t room) {
 // 256), 202 in 128 x 256 (two rounds of 320); 181 take 22 us in 192 x 128
 // over six splits, 29 in 128 x 128 over three, 69 unsplit, and their Q/K/V 46
 // us in 192 x 128 over two splits against 59 in 128 x 256 (a tile that holds
-// every token reads each weight row once).
-struct GemmPlan {
-    const GemmForm *form;
-    int splits;
-    const GemmPairForm *pair;  // two heights instead of form
-    GemmPair cut;
-};
-GemmPlan gemm_plan(const ProjectArgs &a, bool heads, int n_cu, size_t part_floats) {
+// every token reads each weight row once).  With a.hold only partials do, of
+// one slice or several.
+bool plan_gemm(const ProjectArgs &a, bool heads, int n_cu, size_t part_floats, ProductPlan &plan) {
     const int T = a.n_tok, N = a.n_a + a.n_b;
+    if (a.hidden % kGKc != 0 || T > kBigProjMaxTokens || (heads && N % kHeadDim != 0)) return false;
     const int nc = a.hidden / kGKc;
     const double stream_us = 2.0 * a.hidden * (static_cast<double>(N) + T) / 5.0e6;
-    GemmPlan best{};
+    ProductPlan best{};
+    best.form = best.pair = -1;
     double best_us = 0;
-    for (const GemmForm &f : kForms) {
+    for (int i = 0; i < static_cast<int>(std::size(kForms)); ++i) {
+        const GemmForm &f = kForms[i];
         // Row offsets within a tile are 32-bit.
         if (static_cast<uint64_t>(std::max(f.bm, f.bn)) * 2u * static_cast<uint32_t>(a.hidden) > 0xffffffffull) continue;
         if (heads && a.n_a % f.bn != 0) continue;  // a tile never straddles the two weights
         const double tiles = static_cast<double>((N + f.bn - 1) / f.bn) * ((T + f.bm - 1) / f.bm);
         for (int splits = 1; splits <= kGemmMaxSplits && splits <= nc; ++splits) {
-            if (splits == 1 ? !(heads ? f.head : f.out) : !f.part) continue;
+            const bool partial = splits > 1 || a.hold;
+            if (partial ? !f.part : !(heads ? f.head : f.out)) continue;
             const double part = static_cast<double>(splits) * T * N;
-            if (splits > 1 && part > static_cast<double>(part_floats)) break;
+            if (partial && part > static_cast<double>(part_floats)) break;
             const double rounds = static_cast<double>((static_cast<int64_t>(tiles * splits) + n_cu - 1) / n_cu);
             const double walk = rounds * ((nc + splits - 1) / splits) * f.chunk_us;
             // A CU streams its share of the operands: fewer workgroups than
@@ -559,18 +553,23 @@ GemmPlan gemm_plan(const ProjectArgs &a, bool heads, int n_cu, size_t part_float
             const double fill = tiles * splits < n_cu ? n_cu / (tiles * splits) : 1.0;
             const double stream = stream_us * fill;
             double us = 3.0 * rounds + (walk > stream ? walk + 0.1 * stream : stream + 0.1 * walk);
-            if (splits > 1) us += 4.0 + 8.0 * part / 5.0e6;
-            if (!best.form || us < best_us) {
-                best.form = &f;
+            if (partial) us += 4.0 + 8.0 * part / 5.0e6;
+            if (best.form < 0 || us < best_us) {
+                best.form = i;
                 best.splits = splits;
+                best.partial = partial;
                 best_us = us;
             }
         }
     }
+    if (best.form < 0) return false;
+    best.bm = kForms[best.form].bm;
+    best.bn = kForms[best.form].bn;
     // Two heights, where one leaves its last round part empty.
-    for (const GemmPairForm &f : kPairs) {
+    for (int i = 0; i < static_cast<int>(std::size(kPairs)); ++i) {
+        const GemmPairForm &f = kPairs[i];
         const GemmForm &ft = kForms[f.tall], &fl = kForms[f.low];
-        if (!heads || !best.form || best.splits > 1 || a.n_a % ft.bn != 0) break;
+        if (!heads || best.partial || a.n_a % ft.bn != 0) break;
         const int n_rt = N / ft.bn;
         const int64_t round = static_cast<int64_t>(n_cu) * ft.bm;
         const int rounds = static_cast<int>((static_cast<int64_t>(T) * n_rt + round - 1) / round);
@@ -581,26 +580,24 @@ GemmPlan gemm_plan(const ProjectArgs &a, bool heads, int n_cu, size_t part_float
             const double walk = nc * (r * ft.chunk_us + more * fl.chunk_us);
             const double us = 3.0 * (r + more) + (walk > stream_us ? walk + 0.1 * stream_us : stream_us + 0.1 * walk);
             if (us < best_us) {
-                best.pair = &f;
+                best.pair = i;
                 best.cut = cut;
+                best.bm = ft.bm;
+                best.bn = ft.bn;
+                best.low = fl.bm;
                 best_us = us;
             }
         }
     }
-    return best;
+    plan = best;
+    return true;
 }
 
-}  // namespace
-
-hipError_t launch_gemm_project(ProjectArgs &a, bool heads, int n_cu, size_t part_floats, hipStream_t s) {
-    if (a.hidden % kGKc != 0 || a.n_tok > kBigProjMaxTokens || (heads && (a.n_a + a.n_b) % kHeadDim != 0))
-        return hipErrorInvalidValue;
-    const GemmPlan plan = gemm_plan(a, heads, n_cu, part_floats);
-    if (!plan.form) return hipErrorInvalidValue;
-    a.splits = plan.splits;
-    if (plan.pair) return plan.pair->launch(a, plan.cut, s);
-    if (a.splits > 1) return plan.form->launch_part(a, s);
-    return (heads ? plan.form->launch_head : plan.form->launch_out)(a, s);
+hipError_t launch_gemm_project(const ProjectArgs &a, bool heads, const ProductPlan &plan, hipStream_t s) {
+    if (plan.pair >= 0) return kPairs[plan.pair].launch(a, plan.cut, s);
+    const GemmForm &form = kForms[plan.form];
+    if (plan.partial) return form.launch_part(a, s);
+    return (heads ? form.launch_head : form.launch_out)(a, s);
 }
 
 }  // namespace kva

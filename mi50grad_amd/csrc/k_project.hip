@@ -322,32 +322,33 @@ hipError_t launch_stream(const ProjectArgs &a, hipStream_t s) {
     return hipGetLastError();
 }
 
-// The product, between the caller's timing events (if any); `partial` is set
-// when it leaves partials for a finish kernel.
-hipError_t launch_product(ProjectArgs &a, bool heads, int n_cu, size_t part_floats, bool &partial, hipStream_t s) {
+// The product, between the caller's timing events (if any).
+hipError_t launch_product(ProjectArgs &a, bool heads, const ProductPlan &plan, hipStream_t s) {
     if (a.ev_before) {
         const hipError_t e = hipEventRecord(a.ev_before, s);
         if (e != hipSuccess) return e;
     }
-    hipError_t e;
-    if (streams(a)) {
-        partial = true;
-        e = launch_stream(a, s);
-    } else {
-        e = launch_gemm_project(a, heads, n_cu, part_floats, s);
-        partial = a.splits > 1;
-    }
+    a.splits = plan.splits;
+    const hipError_t e = plan.stream ? launch_stream(a, s) : launch_gemm_project(a, heads, plan, s);
     if (e != hipSuccess || !a.ev_after) return e;
     return hipEventRecord(a.ev_after, s);
 }
 
 }  // namespace
 
-hipError_t launch_project(ProjectArgs a, int n_cu, size_t part_floats, hipStream_t s) {
+bool plan_product(const ProjectArgs &a, bool heads, int n_cu, size_t part_floats, ProductPlan &plan) {
+    if (!streams(a)) return plan_gemm(a, heads, n_cu, part_floats, plan);
+    plan = ProductPlan{};
+    plan.stream = plan.partial = true;
+    plan.splits = a.splits;
+    plan.form = plan.pair = -1;
+    return true;
+}
+
+hipError_t launch_project(ProjectArgs a, const ProductPlan &plan, hipStream_t s) {
     if (a.n_tok <= 0) return hipSuccess;
-    bool partial = false;
-    const hipError_t e = launch_product(a, true, n_cu, part_floats, partial, s);
-    if (e != hipSuccess || !partial) return e;
+    const hipError_t e = launch_product(a, true, plan, s);
+    if (e != hipSuccess || !plan.partial) return e;
     const int blocks_per_tok = (2 * a.num_heads + 2 * a.num_kv_heads + 7) / 8;
     const dim3 grid(static_cast<unsigned>(a.n_tok) * blocks_per_tok), block(256);
     if (a.splits <= 2) hipLaunchKernelGGL(proj_finish_kernel<2>, grid, block, 0, s, a);
@@ -356,12 +357,11 @@ hipError_t launch_project(ProjectArgs a, int n_cu, size_t part_floats, hipStream
     return hipGetLastError();
 }
 
-hipError_t launch_out_project(ProjectArgs a, int n_cu, size_t part_floats, hipStream_t s) {
+hipError_t launch_out_project(ProjectArgs a, const ProductPlan &plan, hipStream_t s) {
     if (a.n_tok <= 0) return hipSuccess;
     if (a.n_b != 0 || a.n_a % 16 != 0) return hipErrorInvalidValue;
-    bool partial = false;
-    const hipError_t e = launch_product(a, false, n_cu, part_floats, partial, s);
-    if (e != hipSuccess || !partial) return e;
+    const hipError_t e = launch_product(a, false, plan, s);
+    if (e != hipSuccess || !plan.partial) return e;
     const int64_t threads = static_cast<int64_t>(a.n_tok) * (a.n_a / 8);
     const dim3 grid(static_cast<unsigned>((threads + 255) / 256)), block(256);
     if (a.splits <= 2) hipLaunchKernelGGL(oproj_finish_kernel<2>, grid, block, 0, s, a);

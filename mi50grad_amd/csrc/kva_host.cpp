@@ -88,6 +88,7 @@ struct kva_cache {
     size_t part_floats = 0;     // what it holds
     size_t proj_floats = 0;     // the partials that kva_out_project's refusals are counted in
     int32_t last_proj_path = 0;  // KVA_PROJECT_KERNELS or KVA_PROJECT_PREFILL_GEMM
+    kva::ProductPlan last_product{};  // of the last projection's first launch
     int32_t max_wg = 0;  // decode workgroups the partial workspace can serve
     size_t ws_rows = 0;  // 256-float rows in the decode partial workspace
     int32_t n_cu = 0;
@@ -938,6 +939,22 @@ static int32_t project_splits(const kva_cache *c, int32_t hidden, int32_t n_rows
     return best;
 }
 
+// Whether n elements of fp16 output at `out` overlap m of an operand at `in`.
+static bool overlaps(const void *out, size_t n, const void *in, size_t m) {
+    const auto o = reinterpret_cast<uintptr_t>(out), i = reinterpret_cast<uintptr_t>(in);
+    return out && in && o < i + 2 * m && i < o + 2 * n;
+}
+
+// Tokens a launch of `a` takes.  A held product's partials fit the workspace,
+// and its launches go in token order: out over attn (or q_out over x) of rows
+// no longer than those it overwrites stays right across launches.  At least
+// kProjTokens tokens fit, by the refusals.
+static int32_t tokens_per_launch(const kva_cache *c, const kva::ProjectArgs &a) {
+    if (!a.hold) return kva::kBigProjMaxTokens;
+    const size_t fit = c->part_floats / (static_cast<size_t>(a.n_a) + a.n_b);
+    return static_cast<int32_t>(std::min<size_t>(fit, kva::kBigProjMaxTokens));
+}
+
 static int project_impl(kva_cache *c, int32_t layer, const void *x, int32_t hidden, const void *w_q_fused,
                         const void *w_kv_fused, const void *q_norm_w, const void *k_norm_w, const void *cos_tab,
                         const void *sin_tab, int32_t table_rows, void *q_out, void *q_gate_out, void *kv_out,
@@ -963,7 +980,6 @@ static int project_impl(kva_cache *c, int32_t layer, const void *x, int32_t hidd
     if (c->st_max_pos >= table_rows)
         return fail(KVA_ERR_INVALID_ARG, "RoPE position %d beyond the %d table rows", c->st_max_pos,
                     table_rows);
-    if ((rc = require_device(c))) return rc;
     kva::ProjectArgs a{};
     a.w_a = static_cast<const uint16_t *>(w_q_fused);
     a.w_b = static_cast<const uint16_t *>(w_kv_fused);
@@ -972,29 +988,47 @@ static int project_impl(kva_cache *c, int32_t layer, const void *x, int32_t hidd
     a.hidden = hidden;
     a.splits = project_splits(c, hidden, a.n_a + a.n_b);
     a.part = c->d_proj;
-    a.q_out = static_cast<uint16_t *>(q_out);
-    a.gate_out = static_cast<uint16_t *>(q_gate_out);
-    a.kv_out = static_cast<uint16_t *>(kv_out);
     a.q_w = static_cast<const uint16_t *>(q_norm_w);
     a.k_w = static_cast<const uint16_t *>(k_norm_w);
     a.cos_tab = static_cast<const uint16_t *>(cos_tab);
     a.sin_tab = static_cast<const uint16_t *>(sin_tab);
-    a.k_pool = c->d_k + c->layer_elems * layer;
-    a.v_pool = c->d_v + c->layer_elems * layer;
     a.table = c->d_table;
     a.table_stride = c->cfg.max_blocks_per_seq;
-    a.tok_seq = at<int32_t>(c->d_step, c->off_tseq);
-    a.tok_slot = at<int32_t>(c->d_step, c->off_tslot);
-    a.tok_pos = at<int32_t>(c->d_step, c->off_tpos);
     a.num_heads = c->cfg.num_heads;
     a.num_kv_heads = c->cfg.num_kv_heads;
     a.half_rot = half_rot;
     a.eps = c->cfg.eps;
     a.ev_before = c->kev_before;
     a.ev_after = c->kev_after;
-    a.x = static_cast<const uint16_t *>(x);
-    a.n_tok = c->st_n_tok;
-    KVA_HIP(kva::launch_project(a, c->n_cu, c->part_floats, static_cast<hipStream_t>(stream)));
+    const size_t T = c->st_n_tok, q_row = static_cast<size_t>(c->cfg.num_heads) * kva::kHeadDim,
+                 kv_row = 2 * static_cast<size_t>(c->cfg.num_kv_heads) * kva::kHeadDim, h = hidden;
+    auto over_operand = [&](const void *out, size_t n) {
+        return overlaps(out, n, x, T * h) || overlaps(out, n, w_q_fused, a.n_a * h) ||
+               overlaps(out, n, w_kv_fused, a.n_b * h);
+    };
+    a.hold = over_operand(q_out, T * q_row) || over_operand(q_gate_out, T * q_row) || over_operand(kv_out, T * kv_row);
+    const int32_t per = tokens_per_launch(c, a);
+    a.n_tok = std::min(per, c->st_n_tok);
+    kva::ProductPlan plan{};
+    bool planned = kva::plan_product(a, true, c->n_cu, c->part_floats, plan);
+    c->last_product = plan;
+    if ((rc = require_device(c))) return rc;
+    a.k_pool = c->d_k + c->layer_elems * layer;
+    a.v_pool = c->d_v + c->layer_elems * layer;
+    for (int32_t t0 = 0; t0 < c->st_n_tok; t0 += per) {
+        a.x = static_cast<const uint16_t *>(x) + t0 * h;
+        a.q_out = static_cast<uint16_t *>(q_out) + t0 * q_row;
+        a.gate_out = q_gate_out ? static_cast<uint16_t *>(q_gate_out) + t0 * q_row : nullptr;
+        a.kv_out = kv_out ? static_cast<uint16_t *>(kv_out) + t0 * kv_row : nullptr;
+        a.tok_seq = at<int32_t>(c->d_step, c->off_tseq) + t0;
+        a.tok_slot = at<int32_t>(c->d_step, c->off_tslot) + t0;
+        a.tok_pos = at<int32_t>(c->d_step, c->off_tpos) + t0;
+        if (const int32_t n = std::min(per, c->st_n_tok - t0); n != a.n_tok) {
+            a.n_tok = n;
+            planned = kva::plan_product(a, true, c->n_cu, c->part_floats, plan);
+        }
+        KVA_HIP(planned ? kva::launch_project(a, plan, static_cast<hipStream_t>(stream)) : hipErrorInvalidValue);
+    }
     c->last_proj_path = c->st_n_tok > kva::kProjTokens ? KVA_PROJECT_PREFILL_GEMM : KVA_PROJECT_KERNELS;
     return KVA_OK;
 }
@@ -1002,6 +1036,19 @@ static int project_impl(kva_cache *c, int32_t layer, const void *x, int32_t hidd
 int kva_get_project_path(const kva_cache *c, int32_t *path) {
     if (!c || !path) return fail(KVA_ERR_INVALID_ARG, "NULL argument");
     *path = c->last_proj_path;
+    return KVA_OK;
+}
+
+int kva_get_product_plan(const kva_cache *c, int32_t *tile_tokens, int32_t *low_tokens, int32_t *tile_rows,
+                         int32_t *splits, int32_t *partial) {
+    if (!c || !tile_tokens || !low_tokens || !tile_rows || !splits || !partial)
+        return fail(KVA_ERR_INVALID_ARG, "NULL argument");
+    const kva::ProductPlan &p = c->last_product;
+    *tile_tokens = p.bm;
+    *low_tokens = p.low;
+    *tile_rows = p.bn;
+    *splits = p.splits;
+    *partial = p.partial;
     return KVA_OK;
 }
 
@@ -1312,17 +1359,28 @@ static int out_project_impl(kva_cache *c, const void *attn, int32_t n_tok, int32
     if (static_cast<size_t>(a.splits) * chunk_tok * n_out > c->proj_floats)
         return fail(KVA_ERR_INVALID_ARG, "n_out %d x %lld tokens exceeds the projection workspace (%zu floats)", n_out,
                     static_cast<long long>(chunk_tok), c->proj_floats);
-    if (int rc = require_device(c)) return rc;
     a.part = c->d_proj;
     a.ev_before = c->kev_before;
     a.ev_after = c->kev_after;
-    for (int32_t t0 = 0; t0 < n_tok; t0 += kva::kBigProjMaxTokens) {
+    const size_t out_elems = static_cast<size_t>(n_tok) * n_out;
+    a.hold = overlaps(out, out_elems, attn, static_cast<size_t>(n_tok) * q_dim) ||
+             overlaps(out, out_elems, w_o, static_cast<size_t>(n_out) * q_dim);
+    const int32_t per = tokens_per_launch(c, a);
+    a.n_tok = std::min(per, n_tok);
+    kva::ProductPlan plan{};
+    bool planned = kva::plan_product(a, false, c->n_cu, c->part_floats, plan);
+    c->last_product = plan;
+    if (int rc = require_device(c)) return rc;
+    for (int32_t t0 = 0; t0 < n_tok; t0 += per) {
         const size_t at0 = static_cast<size_t>(t0) * n_out;
         a.x = static_cast<const uint16_t *>(attn) + static_cast<size_t>(t0) * q_dim;
         a.y_out = static_cast<uint16_t *>(out) + at0;
         a.residual = residual ? static_cast<const uint16_t *>(residual) + at0 : nullptr;
-        a.n_tok = std::min(kva::kBigProjMaxTokens, n_tok - t0);
-        KVA_HIP(kva::launch_out_project(a, c->n_cu, c->part_floats, static_cast<hipStream_t>(stream)));
+        if (const int32_t n = std::min(per, n_tok - t0); n != a.n_tok) {
+            a.n_tok = n;
+            planned = kva::plan_product(a, false, c->n_cu, c->part_floats, plan);
+        }
+        KVA_HIP(planned ? kva::launch_out_project(a, plan, static_cast<hipStream_t>(stream)) : hipErrorInvalidValue);
     }
     return KVA_OK;
 }

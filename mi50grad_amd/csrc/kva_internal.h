@@ -76,6 +76,9 @@ struct ProjectArgs {
     int32_t hidden;
     int32_t n_tok;
     int32_t splits;           // of hidden among workgroups
+    // An output overlaps x or a weight: the product goes to partials whole,
+    // so that every operand has been read when the finish kernel writes.
+    bool hold;
     float *part;              // [splits][n_tok][n_a + n_b]
     uint16_t *q_out;          // [T][H][256]: normalised + rotated Q
     uint16_t *gate_out;       // [T][H][256]: Q_gate as projected (nullable)
@@ -103,15 +106,34 @@ struct ProjectArgs {
     // DecodeArgs.
     hipEvent_t ev_before, ev_after;
 };
+// How gemm_pair_kernel cuts its row tiles.
+struct GemmPair {
+    int tall, all;         // workgroups of tall tiles, and of both
+    int heads;             // row tiles of the first kind
+    int hi, lo;            // tall tiles of one row tile of the first kind, of the others
+    int rest_hi, rest_lo;  // the same of the low ones
+};
+// How a product runs: the x-resident form (stream), a tile GEMM or one of two
+// tile heights (pair).  Partial: it leaves `splits` partials for a finish
+// kernel; else the outputs are written.
+struct ProductPlan {
+    bool stream, partial;
+    int splits;
+    int form, pair;   // of the tables in k_gemm.hip (-1: none)
+    GemmPair cut;
+    int bm, bn, low;  // tile tokens and rows (0 with stream), tokens of the low tiles (0: one height)
+};
+// The plan of `a`: heads, the Q/K/V projection, else the O-projection.
 // `a.splits` is the split of the x-resident form; part_floats what a.part
 // holds (the GEMM forms choose their own split from it and the CU count).
-hipError_t launch_project(ProjectArgs a, int n_cu, size_t part_floats, hipStream_t s);
-hipError_t launch_out_project(ProjectArgs a, int n_cu, size_t part_floats, hipStream_t s);
-// The LDS-tiled GEMM of either (k_gemm.hip): heads, the Q/K/V projection;
-// else the O-projection.  Sets a.splits: 1, the outputs are written; more,
-// a.part holds that many partials.  Needs hidden % 64 == 0.
+// False where no form takes it.
+bool plan_product(const ProjectArgs &a, bool heads, int n_cu, size_t part_floats, ProductPlan &plan);
+hipError_t launch_project(ProjectArgs a, const ProductPlan &plan, hipStream_t s);
+hipError_t launch_out_project(ProjectArgs a, const ProductPlan &plan, hipStream_t s);
+// The LDS-tiled GEMMs of both (k_gemm.hip).  Need hidden % 64 == 0.
 constexpr int kBigProjMaxTokens = 1 << 24;
-hipError_t launch_gemm_project(ProjectArgs &a, bool heads, int n_cu, size_t part_floats, hipStream_t s);
+bool plan_gemm(const ProjectArgs &a, bool heads, int n_cu, size_t part_floats, ProductPlan &plan);
+hipError_t launch_gemm_project(const ProjectArgs &a, bool heads, const ProductPlan &plan, hipStream_t s);
 
 // Reference-compatible norm+RoPE on a contiguous [n_heads][head_dim] buffer.
 struct LegacyNormArgs {

@@ -195,6 +195,14 @@ class PagedKVCache:
         _lib.call("kva_get_project_path", self.handle, ctypes.byref(p))
         return {0: "kernels", 1: "prefill_gemm"}[p.value]
 
+    def product_plan(self) -> dict:
+        """The launch of the last project_append or out_project
+        (kva_get_product_plan)."""
+        names = ("tile_tokens", "low_tokens", "tile_rows", "splits", "partial")
+        vals = [ctypes.c_int32() for _ in names]
+        _lib.call("kva_get_product_plan", self.handle, *[ctypes.byref(v) for v in vals])
+        return {n: v.value for n, v in zip(names, vals)}
+
     def out_project(self, attn, n_tok: int, q_dim: int, w_o, n_out: int, out, residual=None,
                     stream=None) -> None:
         """O-projection of n_tok attention rows: out = fp16(attn . w_o^T +
