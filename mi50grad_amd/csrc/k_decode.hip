@@ -1169,13 +1169,16 @@ hipError_t launch_g(const DecodeArgs &a, hipStream_t s) {
     // Sixteen waves hold 256 pieces in flight, where a CU has one workgroup at
     // most (a second round of them costs more: three sequences of 85 pieces
     // 6.9 us, 4.2 with eight waves; one of 256 pieces 5.0 and 5.0, two 4.4 and
-    // 4.6).  Eight hold 128, worth it from about 50 pieces a sequence (four
-    // sequences of 64: 4.5 us, 4.8 with four waves); four hold the rest.
+    // 4.6).  Eight hold 128, worth it where 256 shares come to about 50 pieces
+    // a sequence (four sequences of 64: 4.5 us, 4.8 with four waves); four hold
+    // the rest.  The waves set the order of the sums, so they depend on nothing
+    // that a recorded launch does not know (it has the most shares there can
+    // be, the step it replays may have fewer): the sequences and the heads.
     if (a.few_pieces)
         hipLaunchKernelGGL((combine_kernel<G>), dim3(units), dim3(64 * G), 0, s, a);
     else if (units * G * 4 <= 256)
         hipLaunchKernelGGL((combine_wide_kernel<G, 16>), dim3(units, G, 4), dim3(64 * 16), 0, s, a);
-    else if (a.n_wg > 48 * a.n_seqs)
+    else if (48 * a.n_seqs < 256)
         hipLaunchKernelGGL((combine_wide_kernel<G, 8>), dim3(units, G, 4), dim3(64 * 8), 0, s, a);
     else
         hipLaunchKernelGGL((combine_wide_kernel<G, 4>), dim3(units, G, 4), dim3(64 * 4), 0, s, a);

@@ -54,6 +54,16 @@ def test_graph_replay_matches_eager(device, lengths, split, fused):
     _replay(device, lengths, split, fused, steps=21, same_outputs=True, other_shape=True)
 
 
+# Sequences of more than 16 pieces, merged by 16 waves (one sequence, 48), 8
+# (three: 38 and 69 pieces, over fewer shares than a recorded launch has) and 4
+# (six: 57 and 44).
+@pytest.mark.parametrize("lengths,split", [([760], 16), ([600, 5, 77], 16), ([1100, 300, 300], 0),
+                                           ([900, 5, 700, 30, 40, 77], 16)])
+def test_graph_replay_many_pieces(device, lengths, split):
+    say(f"graph replay many pieces lengths={lengths} split={split}")
+    _replay(device, lengths, split, False, steps=4, same_outputs=True, other_shape=False)
+
+
 @pytest.mark.parametrize("fused", [False, True])
 def test_graph_whole_form_past_64_pages(device, fused):
     """A step recorded in the whole-sequence form (longest sequence 1021
