@@ -667,8 +667,8 @@ __device__ __forceinline__ size_t piece_row(const DecodeArgs &a, const Pieces &p
 
 // Dims d0 .. d0+3 of the merge of at most kCombineChunk pieces by one wave,
 // every load requested before any is used; lt: the sum of probabilities.
-// Both combine forms merge such a sequence here, so a recorded step (always
-// the wide form) gives the bits of the ordinary one.
+// Every combine form merges such a sequence here, so a recorded step (never
+// combine_kernel) gives the bits of the ordinary one.
 template <int G>
 __device__ __forceinline__ float4_t merge_few(const DecodeArgs &a, const Pieces &p, int h, int g, int d0, int lane,
                                               float &lt) {
@@ -728,6 +728,63 @@ __global__ __launch_bounds__(64 * G) void combine_kernel(DecodeArgs a) {
     *reinterpret_cast<uint2 *>(a.out + (static_cast<size_t>(b) * a.num_heads + h * G + g) * kHeadDim + 4 * lane) = y;
 }
 
+// The running merge of some pieces' partials: (reference max in log2 units,
+// sum of probabilities, four dims).  Both wide forms fold and join through
+// these, with the products and sums spelled out, so they give the same bits.
+struct Merge {
+    float big = -INFINITY, lt = 0.0f;
+    float4_t at = float4_t{0.f, 0.f, 0.f, 0.f};
+
+    // Pieces (m, l) = ml[k], acc v[k]; m = -inf: none, weighs nothing.
+    template <int N>
+    __device__ __forceinline__ void fold(const float2 (&ml)[N], const float4_t (&v)[N]) {
+        float nb = big;
+#pragma unroll
+        for (int k = 0; k < N; ++k) nb = fmaxf(nb, ml[k].x);
+        if (nb == -INFINITY) return;
+        const float keep = __builtin_amdgcn_exp2f(big - nb);  // 0 before any
+        lt *= keep;
+        at *= keep;
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const float c = __builtin_amdgcn_exp2f(ml[k].x - nb);
+            lt = fmaf(c, ml[k].y, lt);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) at[e] = fmaf(c, v[k][e], at[e]);
+        }
+        big = nb;
+    }
+    __device__ __forceinline__ void join(const Merge &o) {
+        const float nb = fmaxf(big, o.big);
+        const float mu = nb == -INFINITY ? 0.0f : nb;
+        const float c0 = __builtin_amdgcn_exp2f(big - mu), c1 = __builtin_amdgcn_exp2f(o.big - mu);
+        lt = fmaf(o.lt, c1, lt * c0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) at[e] = fmaf(o.at[e], c1, at[e] * c0);
+        big = nb;
+    }
+};
+
+// The merges of a workgroup's NW waves, LP lanes each, through LDS: wave w's
+// in w_acc[w * LP + lane] and w_ml[w].
+template <int NW, int LP>
+__device__ __forceinline__ void join_waves(Merge &m, const float4 *w_acc, const float2 *w_ml, int lane) {
+    float mm = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) mm = fmaxf(mm, w_ml[w].x);
+    m.lt = 0.0f;
+    m.at = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        const float c = __builtin_amdgcn_exp2f(w_ml[w].x - mm);  // 0 for a wave without pieces
+        const float4 x = w_acc[w * LP + lane];
+        m.lt = fmaf(w_ml[w].y, c, m.lt);
+        const float4_t xv = {x.x, x.y, x.z, x.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) m.at[e] = fmaf(c, xv[e], m.at[e]);
+    }
+}
+
 // combine_wide_kernel (any number of pieces: one long sequence over every CU
 // has 256): a workgroup per (sequence, query head, quarter of the head's
 // dims).  A wave takes four pieces per load instruction, 16 lanes x 4 dims
@@ -765,8 +822,7 @@ __global__ __launch_bounds__(64 * NW) void combine_wide_kernel(DecodeArgs a) {
         if (lane < 16) store(o, l);
         return;
     }
-    float big = -INFINITY, lt = 0.0f;
-    float4_t at = float4_t{0.f, 0.f, 0.f, 0.f};
+    Merge m;
     for (int i0 = 4 * wave; i0 < p.n; i0 += 4 * NW * kDepth) {
         float2 ml[kDepth];
         float4_t v[kDepth];
@@ -779,53 +835,96 @@ __global__ __launch_bounds__(64 * NW) void combine_wide_kernel(DecodeArgs a) {
             v[k] = *reinterpret_cast<const float4_t *>(a.ws_acc + row * kHeadDim + d0);
             if (!ok) ml[k].x = -INFINITY;
         }
-        float nb = big;
-#pragma unroll
-        for (int k = 0; k < kDepth; ++k) nb = fmaxf(nb, ml[k].x);
-        if (nb > -INFINITY) {  // this lane group has a piece
-            const float keep = __builtin_amdgcn_exp2f(big - nb);  // 0 before any
-            lt *= keep;
-            at *= keep;
-#pragma unroll
-            for (int k = 0; k < kDepth; ++k) {
-                const float c = __builtin_amdgcn_exp2f(ml[k].x - nb);  // 0 past the last piece
-                lt += c * ml[k].y;
-                at += c * v[k];
-            }
-            big = nb;
-        }
+        m.fold(ml, v);
     }
-    // The four lane groups, then the waves.
+    // The four lane groups (lane group 0's order of them), then the waves.
 #pragma unroll
     for (int o = 16; o <= 32; o <<= 1) {
-        const float ob = __shfl_xor(big, o), ol = __shfl_xor(lt, o);
-        float4_t oa;
+        Merge other;
+        other.big = __shfl_xor(m.big, o);
+        other.lt = __shfl_xor(m.lt, o);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) oa[c] = __shfl_xor(at[c], o);
-        const float nb = fmaxf(big, ob);
-        const float mu = nb == -INFINITY ? 0.0f : nb;
-        const float c0 = __builtin_amdgcn_exp2f(big - mu), c1 = __builtin_amdgcn_exp2f(ob - mu);
-        lt = lt * c0 + ol * c1;
-        at = at * c0 + oa * c1;
-        big = nb;
+        for (int c = 0; c < 4; ++c) other.at[c] = __shfl_xor(m.at[c], o);
+        m.join(other);
     }
-    if (lane < 16) w_acc[wave * 16 + lane] = make_float4(at[0], at[1], at[2], at[3]);
-    if (lane == 0) w_ml[wave] = make_float2(big, lt);
+    if (lane < 16) w_acc[wave * 16 + lane] = make_float4(m.at[0], m.at[1], m.at[2], m.at[3]);
+    if (lane == 0) w_ml[wave] = make_float2(m.big, m.lt);
     __syncthreads();
     if (threadIdx.x >= 16) return;
-    float mm = -INFINITY;
+    join_waves<NW, 16>(m, w_acc, w_ml, lane);
+    store(m.at, m.lt);
+}
+
+// The same merge as combine_wide_kernel's of four waves, bit for bit, with a
+// workgroup per (sequence, query head) and the whole head in a wave.  A
+// recorded launch cannot know that every sequence has few pieces, and at many
+// sequences the start of the wide form's workgroups, most of which find one
+// wave's work or none, is all its time: 64 sequences of 1030 to 2000 rows
+// replay with a merge of 15.7 us in it and 8.2 in this form (eagerly, with
+// combine_kernel, 4.9).  Held to five waves a SIMD it spills (one sequence of
+// 16000 rows among 31 of 200: a layer 36.4 us as it is, 38.9 so).
+template <int G>
+__global__ __launch_bounds__(256) void combine_head_kernel(DecodeArgs a) {
+    constexpr int NW = 4, kDepth = 4;
+    __shared__ float4 w_acc[NW * 64];
+    __shared__ float2 w_ml[NW];
+    const int u = blockIdx.x;
+    const int g = blockIdx.y;
+    const int hkv = a.num_kv_heads;
+    const int b = u / hkv;
+    const int h = u - b * hkv;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    Pieces p;
+    if (!find_pieces(a, b, p)) return;  // uniform over the workgroup
+    float4_t o;
+    float l;
+    if (p.n <= kCombineChunk) {
+        if (wave != 0) return;
+        o = merge_few<G>(a, p, h, g, 4 * lane, lane, l);
+    } else {
+        // Group s: the pieces that lane group s of the quarter form takes.
+        Merge m[4];
+        for (int i0 = 4 * wave; i0 < p.n; i0 += 4 * NW * kDepth) {
+            // Lane j holds the (m, l) of piece j of these sixteen: piece
+            // i0 + 4 NW (j / 4) + j % 4.
+            const int ij = i0 + 4 * NW * ((lane >> 2) & 3) + (lane & 3);
+            float2 mine = make_float2(-INFINITY, 0.0f);
+            if (ij < p.n) mine = *reinterpret_cast<const float2 *>(a.ws_ml + piece_row<G>(a, p, ij, h, g) * 2);
+            float4_t v[4][kDepth];
 #pragma unroll
-    for (int w = 0; w < NW; ++w) mm = fmaxf(mm, w_ml[w].x);
-    lt = 0.0f;
-    at = float4_t{0.f, 0.f, 0.f, 0.f};
+            for (int k = 0; k < kDepth; ++k)
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
-        const float c = __builtin_amdgcn_exp2f(w_ml[w].x - mm);  // 0 for a wave without pieces
-        const float4 x = w_acc[w * 16 + lane];
-        lt += w_ml[w].y * c;
-        at += c * float4_t{x.x, x.y, x.z, x.w};
+                for (int s = 0; s < 4; ++s) {
+                    const int i = i0 + 4 * NW * k + s;
+                    v[s][k] = *reinterpret_cast<const float4_t *>(
+                        a.ws_acc + piece_row<G>(a, p, i < p.n ? i : 0, h, g) * kHeadDim + 4 * lane);
+                }
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                float2 ml[kDepth];
+#pragma unroll
+                for (int k = 0; k < kDepth; ++k) {
+                    ml[k].x = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mine.x), 4 * k + s));
+                    ml[k].y = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mine.y), 4 * k + s));
+                }
+                m[s].fold(ml, v[s]);
+            }
+        }
+        m[0].join(m[1]);
+        m[2].join(m[3]);
+        m[0].join(m[2]);
+        w_acc[wave * 64 + lane] = make_float4(m[0].at[0], m[0].at[1], m[0].at[2], m[0].at[3]);
+        if (lane == 0) w_ml[wave] = make_float2(m[0].big, m[0].lt);
+        __syncthreads();
+        if (wave != 0) return;
+        join_waves<NW, 64>(m[0], w_acc, w_ml, lane);
+        o = m[0].at;
+        l = m[0].lt;
     }
-    store(at, lt);
+    const float inv = 1.0f / l;
+    *reinterpret_cast<uint2 *>(a.out + (static_cast<size_t>(b) * a.num_heads + h * G + g) * kHeadDim + 4 * lane) =
+        out_fp16x4(o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv, gate_of(a, b, h * G + g, lane));
 }
 
 // Query heads a workgroup from which whole_kernel walks pages: where the
@@ -1166,20 +1265,29 @@ hipError_t launch_g(const DecodeArgs &a, hipStream_t s) {
     hipLaunchKernelGGL(decode_mfma_kernel<G>, dim3(a.n_wg, a.num_kv_heads / hpw), dim3(64 * hpw), 0, s, a);
     if ((e = hipGetLastError()) != hipSuccess || (e = mark(a.ev_after, s)) != hipSuccess) return e;
     const int units = a.n_seqs * a.num_kv_heads;
-    // Sixteen waves hold 256 pieces in flight, where a CU has one workgroup at
-    // most (a second round of them costs more: three sequences of 85 pieces
-    // 6.9 us, 4.2 with eight waves; one of 256 pieces 5.0 and 5.0, two 4.4 and
-    // 4.6).  Eight hold 128, worth it where 256 shares come to about 50 pieces
-    // a sequence (four sequences of 64: 4.5 us, 4.8 with four waves); four hold
+    // Waves by the pieces that 256 shares come to.  Sixteen hold 256 in flight:
+    // one or two sequences, where a CU has one workgroup at most (a second
+    // round of them costs more: three sequences of 85 pieces 6.9 us, 4.2 with
+    // eight waves; one of 256 pieces 5.0 and 5.0, two 4.4 and 4.6).  Eight hold
+    // 128: up to five sequences (four of 64 pieces 4.5 us, 4.8 with four
+    // waves), and more where the workgroups are few (six query heads: five
+    // sequences of up to 3000 rows 13.0 us a layer, 13.4 with sixteen waves,
+    // 12.8 with four; six, one of 16000 rows, 15.1, 14.9 and 16.3).  Four hold
     // the rest.  The waves set the order of the sums, so they depend on nothing
     // that a recorded launch does not know (it has the most shares there can
     // be, the step it replays may have fewer): the sequences and the heads.
+    // combine_head_kernel takes a recorded launch from where the wide form
+    // would start some five workgroups a CU: replays of 16 sequences of 1030 to
+    // 2000 rows 31.1 us a layer, 31.8 in the wide form, of 32 47.6 and 51.5; of
+    // 12 27.0 in both, and 35.3 against 34.0 with one of 16000 rows.
     if (a.few_pieces)
         hipLaunchKernelGGL((combine_kernel<G>), dim3(units), dim3(64 * G), 0, s, a);
-    else if (units * G * 4 <= 256)
+    else if (a.n_seqs <= 2 && units * G * 4 <= 256)
         hipLaunchKernelGGL((combine_wide_kernel<G, 16>), dim3(units, G, 4), dim3(64 * 16), 0, s, a);
-    else if (48 * a.n_seqs < 256)
+    else if (a.n_seqs <= 5 || units * G * 4 <= 256)
         hipLaunchKernelGGL((combine_wide_kernel<G, 8>), dim3(units, G, 4), dim3(64 * 8), 0, s, a);
+    else if (a.dyn && units * G * 4 > 1280)
+        hipLaunchKernelGGL((combine_head_kernel<G>), dim3(units, G), dim3(64 * 4), 0, s, a);
     else
         hipLaunchKernelGGL((combine_wide_kernel<G, 4>), dim3(units, G, 4), dim3(64 * 4), 0, s, a);
     return hipGetLastError();

@@ -56,9 +56,11 @@ def test_graph_replay_matches_eager(device, lengths, split, fused):
 
 # Sequences of more than 16 pieces, merged by 16 waves (one sequence, 48), 8
 # (three: 38 and 69 pieces, over fewer shares than a recorded launch has) and 4
-# (six: 57 and 44).
+# (six: 57 and 44; fourteen, where the recorded launch merges whole heads: 94,
+# past one pass of the waves, 57, 16 and fewer).
 @pytest.mark.parametrize("lengths,split", [([760], 16), ([600, 5, 77], 16), ([1100, 300, 300], 0),
-                                           ([900, 5, 700, 30, 40, 77], 16)])
+                                           ([900, 5, 700, 30, 40, 77], 16),
+                                           ([1500, 900, 250, 256, 7, 20, 33, 64, 90, 15, 16, 17, 300, 1030], 16)])
 def test_graph_replay_many_pieces(device, lengths, split):
     say(f"graph replay many pieces lengths={lengths} split={split}")
     _replay(device, lengths, split, False, steps=4, same_outputs=True, other_shape=False)
