@@ -239,22 +239,44 @@ __device__ __forceinline__ uint2 pack_out4(float o0, float o1, float o2, float o
     return make_uint2(pack_h2(o0, o1), pack_h2(o2, o3));
 }
 
+// 1/(1+exp(-g)) of an fp16 value g in [-kGateClamp, kGateClamp] in float32, to
+// no more error than expf and an IEEE division: over every gate above -30 (below,
+// any fp16 output is 0) at most 1.17e-7 of the value and 1.62e-8 on average, 1.20e-7
+// and 2.24e-8 with those.  (v_exp_f32 of g times a rounded log2(e) is off by
+// up to 1.77e-6, the argument's rounding growing with |g|.)  log2(e) goes in
+// two parts, of which the first has 13 bits, so its product with g is exact;
+// the second's factor is 1 + t.  r, the reciprocal of 1 + e, takes the
+// reciprocal's error and the factor in one step: e r is 1 - r to its rounding.
+constexpr float kGateClamp = 87.5f;  // exp and its reciprocal stay finite
+__device__ __forceinline__ float sigmoid(float g) {
+    constexpr double kLog2e = 1.4426950408889634, kHi = 5909.0 / 4096.0;
+    constexpr double kLo = (kLog2e - kHi) * 0.6931471805599453;  // as a power of e
+    const float e = __builtin_amdgcn_exp2f(g * static_cast<float>(-kHi));
+    const float t = g * fmaf(g, static_cast<float>(0.5 * kLo * kLo), static_cast<float>(-kLo));
+    const float r = __builtin_amdgcn_rcpf(1.0f + e), u = 1.0f - r;
+    const float q = fmaf(-u, t, fmaf(-e, r, u));
+    return fmaf(r, fmaf(q, q, q), r);
+}
+
 // The output gate on four fp16 attention outputs: each is multiplied by
 // 1/(1+exp(-g)) in float32 and rounded once more (sigmoid_mul.hip:10-22
 // applied to the attention output, engine.py:2055-2056 after decode and
-// :3120-3121 after prefill), so the fused result equals the reference's two
-// launches.  exp and the reciprocal are the hardware's (v_exp_f32,
-// v_rcp_f32, 1 ulp each): the float32 error, about 1e-6, stays far below the
-// fp16 rounding.  expf and an IEEE division are some 40 instructions per
-// value and made the gate 43 of the 174 us of a prefill of 4 x 512 tokens.
+// :3120-3121 after prefill), so the fused result is within one fp16 ulp of the
+// reference's two launches.  Infinite gates give the output and 0, NaN gives
+// NaN (the clamps propagate it).  With expf and the division, some 40
+// instructions per value, the gate was 43 of the 174 us of a prefill of 4 x
+// 512 tokens.
 __device__ __forceinline__ uint2 gate4(uint2 o, uint2 gw) {
-    const float g[4] = {lo_f(gw.x), hi_f(gw.x), lo_f(gw.y), hi_f(gw.y)};
-    const float a[4] = {lo_f(o.x), hi_f(o.x), lo_f(o.y), hi_f(o.y)};
-    float r[4];
+    const half2_t hi = {static_cast<_Float16>(kGateClamp), static_cast<_Float16>(kGateClamp)};
+    const uint32_t w[2] = {gw.x, gw.y}, ow[2] = {o.x, o.y};
+    uint32_t y[2];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-        r[i] = a[i] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g[i] * -1.4426950408889634f));
-    return pack_out4(r[0], r[1], r[2], r[3]);
+    for (int i = 0; i < 2; ++i) {
+        const half2_t c = __builtin_elementwise_maximum(
+            __builtin_elementwise_minimum(__builtin_bit_cast(half2_t, w[i]), hi), -hi);
+        y[i] = pack_h2(lo_f(ow[i]) * sigmoid(static_cast<float>(c.x)), hi_f(ow[i]) * sigmoid(static_cast<float>(c.y)));
+    }
+    return make_uint2(y[0], y[1]);
 }
 
 // Four attention output dims as fp16, through the gate at g4 (8-byte

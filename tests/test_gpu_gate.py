@@ -156,3 +156,56 @@ def test_multi_query_gated(device, tree):
         assert max_err(g[s], orc.sigmoid_gate(att.astype(np.float16), gate[s])) <= TOL, b
         t += chunk[b]
     cache.destroy()
+
+
+@pytest.mark.parametrize("path", ["decode", "prefill", "combine"])
+def test_gate_over_the_fp16_range(device, path):
+    """The gate's float32 error at every size of gate.  A sequence of one row
+    (combine: 40 equal V rows, cut into pieces) returns its V row a exactly,
+    so the gated output is fp16 of a / (1 + exp(-g)) in float32: exp and its
+    argument within 2.5 x 2^-24 of the value, the sum, the reciprocal and the
+    product half an ulp (2^-24) each, 5.5 x 2^-24 together.  It must be the
+    rounding of some value within 6 x 2^-24 of the exact one (exp of g times a
+    log2(e) rounded to float32 is off by up to 30 x 2^-24).  Infinite gates give
+    a and 0, NaN gives NaN."""
+    rng = np.random.default_rng({"decode": 1, "prefill": 2, "combine": 3}[path])
+    B, L = 64, 40 if path == "combine" else 1
+    say(f"gate over the fp16 range, {path}")
+    pages = (L + 15) // 16
+    cache, kr, vr = build_cache([L] * B, [[b * pages + i for i in range(pages)] for b in range(B)], extra_rows=0,
+                                rng=rng)
+    power = rng.uniform(-14, 15.9, (2, B, HKV, D)).max(axis=0)
+    a = (rng.choice([-1.0, 1.0], power.shape) * 2.0 ** power).astype(np.float16)
+    _, vp = cache.layer_pools(0)
+    image = np.repeat(a[:, None], 16 * pages, axis=1)  # pages in order: every row of a sequence is its a
+    _lib.call("kva_memcpy_h2d", vp, np.ascontiguousarray(image).ctypes.data, image.nbytes)
+    for b in range(B):
+        cache.set_len(b, L - 1)
+    # Any gate, and more where exp(-g) is large and the output still normal.
+    gate = rng.integers(0, 1 << 16, (B, H, D)).astype(np.uint16).view(np.float16)
+    gate = np.where(rng.random((B, H, D)) < 0.3, gate, rng.uniform(-22, -4, (B, H, D)).astype(np.float16))
+    q = rng.standard_normal((B, H, D), dtype=np.float32).astype(np.float16)
+    dq, dg = device.array(q), device.array(gate)
+    plain, gated = device.empty((B, H, D), np.float16), device.empty((B, H, D), np.float16)
+    if path == "combine":
+        cache.set_decode_split(16)
+    cache.begin_step(list(range(B)), [1] * B)
+    run = cache.prefill if path == "prefill" else cache.decode
+    run(0, dq, plain)
+    run(0, dq, gated, gate=dg)
+    device.synchronize()
+    p, got, rows = plain.numpy(), gated.numpy(), np.repeat(a, H // HKV, axis=1)
+    if path == "combine":
+        assert ulps(p, rows).max() <= 1  # three pieces' sums over their weights
+    else:
+        assert np.array_equal(p.view(np.uint16), rows.view(np.uint16))
+    g, x = gate.astype(np.float64), p.astype(np.float64)
+    with np.errstate(over="ignore", invalid="ignore"):
+        v = x / (1.0 + np.exp(-g))
+        e = 6 * 2.0 ** -24
+        lo, hi = (v * (1 - e)).astype(np.float16), (v * (1 + e)).astype(np.float16)
+    nan = np.isnan(g)
+    assert np.isnan(got[nan]).all()
+    ok = (got >= np.minimum(lo, hi)) & (got <= np.maximum(lo, hi))
+    assert ok[~nan].all(), (int((~ok[~nan]).sum()), gate[~nan][~ok[~nan]][:8])
+    cache.destroy()
