@@ -207,6 +207,10 @@ int kva_get_project_path(const kva_cache *cache, int32_t *path);
  * into, and whether fp32 partials went to a finish kernel.                 */
 int kva_get_product_plan(const kva_cache *cache, int32_t *tile_tokens, int32_t *low_tokens,
                          int32_t *tile_rows, int32_t *splits, int32_t *partial);
+/* The query tile of the current step's kva_prefill and kva_tree_verify: MFMA
+ * row tiles per wave (two for steps with enough keys per workgroup) and the
+ * new tokens of a unit.                                                     */
+int kva_get_query_tile(const kva_cache *cache, int32_t *row_tiles, int32_t *tokens);
 /* Output projection of the (gated) attention rows, the consumer of
  * kva_decode_gated: out[t] = fp16(attn[t] . W_o^T + residual[t]) for
  * t < n_tok, accumulated in fp32 and rounded once after the residual add.

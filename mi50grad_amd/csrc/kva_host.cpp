@@ -1052,6 +1052,14 @@ int kva_get_product_plan(const kva_cache *c, int32_t *tile_tokens, int32_t *low_
     return KVA_OK;
 }
 
+int kva_get_query_tile(const kva_cache *c, int32_t *row_tiles, int32_t *tokens) {
+    if (!c || !row_tiles || !tokens) return fail(KVA_ERR_INVALID_ARG, "NULL argument");
+    if (!c->step_valid) return fail(KVA_ERR_STATE, "no step begun (kva_step_begin)");
+    *row_tiles = c->st_mq_nt;
+    *tokens = c->st_mq_q;
+    return KVA_OK;
+}
+
 int kva_set_decode_split(kva_cache *c, int32_t split_tokens) {
     if (!c) return fail(KVA_ERR_INVALID_ARG, "cache is NULL");
     if (split_tokens < 0 || split_tokens % kva::kSplitQuantum != 0)

@@ -203,6 +203,13 @@ class PagedKVCache:
         _lib.call("kva_get_product_plan", self.handle, *[ctypes.byref(v) for v in vals])
         return {n: v.value for n, v in zip(names, vals)}
 
+    def query_tile(self) -> tuple[int, int]:
+        """Row tiles per wave and new tokens of a unit in the current step's
+        prefill and tree_verify (kva_get_query_tile)."""
+        n, t = ctypes.c_int32(), ctypes.c_int32()
+        _lib.call("kva_get_query_tile", self.handle, ctypes.byref(n), ctypes.byref(t))
+        return n.value, t.value
+
     def out_project(self, attn, n_tok: int, q_dim: int, w_o, n_out: int, out, residual=None,
                     stream=None) -> None:
         """O-projection of n_tok attention rows: out = fp16(attn . w_o^T +

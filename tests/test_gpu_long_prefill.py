@@ -34,6 +34,7 @@ def test_two_tile_prefill(device, heads, kv_heads, prefix, chunk):
     dq, dg = device.array(q), device.array(gate)
     plain, gated = device.empty((T, heads, D), np.float16), device.empty((T, heads, D), np.float16)
     cache.begin_step(list(range(B)), chunk)
+    assert cache.query_tile() == (2, 256 // (heads // kv_heads))
     cache.prefill(0, dq, plain)
     cache.prefill(0, dq, gated, gate=dg)
     device.synchronize()

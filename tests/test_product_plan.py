@@ -55,3 +55,24 @@ def test_project_outputs_over_x_go_through_partials(n_new):
     beside = project_plan(c, n_new, 6144, q_out=X + n_new * 6144 * 2)
     assert beside == project_plan(c, n_new, 6144)
     c.destroy()
+
+
+def test_query_tile_of_a_step():
+    """Two row tiles per wave from 48 blocks of 64 keys a workgroup in one-tile
+    units (256 workgroups: 12288 blocks), causal steps of eight waves only."""
+    c = PagedKVCache(n_layers=1, max_seqs=2, max_blocks=8192, max_blocks_per_seq=4096, max_step_tokens=4096,
+                     host_only=True)
+    # 24 tiles of 21 tokens, four heads: 128 blocks a unit are 12288.
+    for rows, tiles in ((127 * 64 - 252, 2), (127 * 64 - 253, 1)):
+        c.set_len(0, 0)
+        c.reserve(0, rows)
+        c.set_len(0, rows)
+        c.begin_step([0], [504])
+        assert c.query_tile() == (tiles, 42 if tiles == 2 else 21), rows
+    c.reserve(0, 60100)
+    c.set_len(0, 60000)
+    c.begin_step([0], [10], tree_bits=[1 << i for i in range(10)])
+    assert c.query_tile() == (1, 10)  # four waves of 16 rows, 6 heads a group
+    c.begin_step([0], [63], tree_bits=[1 << i for i in range(63)])
+    assert c.query_tile() == (1, 21)
+    c.destroy()
