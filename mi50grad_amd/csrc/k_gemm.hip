@@ -520,8 +520,10 @@ GemmPair pair_tiles(int T, int n_rt, int bm, int bm_low, int64_t room) {
 // workgroups, and 17.7 over six, 240); a split adds its partials, written and read back, and the finish launch.  The
 // estimate is within 15 % of the measured times it was fitted to (64 to 2048
 // tokens of 5120 -> 14336 and 6144 -> 5120, and their halves and quarters):
-// 2048 tokens of 6144 -> 5120 take 137 us in 128 x 320 tiles (one round of
-// 256), 202 in 128 x 256 (two rounds of 320); 181 take 22 us in 192 x 128
+// 2048 tokens of 6144 -> 5120 take 124 us in 128 x 320 tiles (one round of
+// 256), 162 in 192 x 128 (two rounds); over hidden 1536 to 6144, 3072 to 7168
+// rows and 1300 to 4096 tokens the 128 x 320 tile takes 10 to 28 % less than
+// the next best wherever it is chosen: its rounds come out full; 181 take 22 us in 192 x 128
 // over six splits, 29 in 128 x 128 over three, 69 unsplit, and their Q/K/V 46
 // us in 192 x 128 over two splits against 59 in 128 x 256 (a tile that holds
 // every token reads each weight row once).  With a.hold only partials do, of

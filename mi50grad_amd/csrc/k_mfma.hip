@@ -130,9 +130,11 @@ __device__ __forceinline__ Unit load_unit(const MultiQueryArgs &a, int u, int b)
     return x;
 }
 
-// Page of this wave's keys of block g of unit un (see issue_block).  (Read
-// a block ahead, at the end of the previous block, it measured 10 % slower
-// on config 4.)
+// Page of this wave's keys of block g of unit un (see issue_block), by a
+// scalar load: the four-stage ring's.  (Read a block ahead there, at the end
+// of the previous block, it measured 10 % slower: the scalar load in flight
+// makes every LDS wait of the block drain.  The two-stage ring reads it ahead
+// by a vector load, page_ahead in mq_kernel.)
 template <int WAVES, int KEYS>
 __device__ __forceinline__ int block_page(const Unit &un, int g, bool on, int wv) {
     const int key0 = (g - un.ub) * KEYS + KEYS / WAVES * wv;
@@ -140,7 +142,7 @@ __device__ __forceinline__ int block_page(const Unit &un, int g, bool on, int wv
 }
 
 // Issue this wave's share of block g of unit un into LDS stage `st`: keys
-// kPer*wv .. kPer*wv + kPer-1 of the block (kPer = 32/WAVES, within one
+// kPer*wv .. kPer*wv + kPer-1 of the block (kPer = KEYS/WAVES, within one
 // page), K and V, one 1 KB load per two keys each (lane l writes granule
 // l%32 of key 2i + l/32).  Keys past the sequence read its last key (finite
 // data; the mask drops them).  A disabled issue (past the workgroup's share)
@@ -209,8 +211,10 @@ __device__ __forceinline__ int mq_share_of(int i, int W) {
 // (over 100 cycles) for every 16 to 32 cycles of products.  The scheduling
 // barriers pin the order; a ring of operands holds the reads in flight.
 // Two tiles per wave, 2048 tokens after 16400: 886 us unpinned, 798 with three
-// ahead, 808 with two and 813 with four (more registers than there are); one
-// tile per wave 1050 -> 959.
+// ahead, 808 with two and 813 with four; one tile per wave 1050 -> 959.  Two
+// tiles per wave have no register to spare: 36, 40 and 52 spill with two, three
+// and four ahead, none of them inside the products (the unit's start and end,
+// the page of the next block).
 constexpr int kQkAhead = 3, kPvAhead = 3;
 
 template <int NT, int WAVES, bool TREE, int KEYS>

@@ -311,9 +311,13 @@ constexpr int mq_keys_for(int waves, bool tree_plan) { return (waves == 8 && !tr
 // blocks more than it has: the cost of starting and ending a unit (its query
 // rows, its gate and output), so a share full of short units gets fewer
 // blocks.  Unit u's blocks sit at positions [mq_pre[u] + cost, mq_pre[u+1]).
-// Counted as 2, 3, 4 and 5 blocks of 64 keys, 4 x 512 gated tokens after 46
-// to 1655 cached rows took 124, 119, 114 and 121 us; blocks of 32 keys (each
-// half the time, so half the cost would do) 4 as well.
+// Counted as 2, 3, 4, 5 and 6 blocks, append and attention of a layer: 4 x 512
+// tokens after up to 2048 rows 177, 168, 164, 162 and 163 us; 2048 from empty
+// 145, 137, 136, 137 and 139, after 16400 rows 900, 900, 881, 887 and 885; 16 x
+// 128 from empty 79, 80, 73, 73 and 73; 2 x 1000 after 3000 266, 262, 262, 266
+// and 267; in blocks of 32 keys (trees) 64 of nine nodes on up to 1000 rows 165,
+// 165, 161, 161 and 164, 8 on up to 3000 52.8, 52.4, 51.4, 51.9 and 52.0.  Of
+// sixteen such shapes four is within 2 % of the best on each.
 constexpr int kMqUnitCost = 4;
 constexpr int kMqMaxGroup = 8;    // largest GQA group of the multi-query kernel
 constexpr int kMqCutWords = 8;    // int32 words of a cut-unit record (6 used)

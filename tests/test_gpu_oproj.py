@@ -7,7 +7,7 @@ oracle (oracle.out_project).
 * Random N(0,1) inputs: within one fp16 ulp plus 2^-13 of the correctly
   rounded result (fp32 accumulation in another order than the reference's),
   and equal to it for almost every element; in place (residual = out).
-* The config-3 shape (32 rows, q_dim 6144, n_out 5120), chunking past 64
+* The config-3 shape (32 rows, q_dim 6144, n_out 5120), more than 64
   rows, the x-resident LDS form (q_dim 5120, n_out 10240, <= 32 rows), and
   the validation errors.
 """

@@ -9,11 +9,11 @@ append, against the oracle's producer (oracle.project_append).
   gemv_fp16_v2.hip:22-85); the
   cache's K row is bit-exactly the norm + RoPE of the projected K and its V
   row the projected V; decode over the result within 2e-3 of fp32.
-* Chunking (steps of more than 64 tokens), the hidden sizes that select 1, 2
-  and 4 splits, one-token steps, and the validation errors.
-* Prefill-sized steps (more than 64 tokens) go through the prefill GEMM
-  (tiles of 256 tokens x one head, the norm/RoPE/append epilogue fused): the
-  same contract (bit-exact on exact inputs, within one ulp plus the
+* Steps around 64 tokens, small and large hidden sizes, one-token steps, and
+  the validation errors.
+* Prefill-sized steps (more than 64 tokens) go through the GEMM tiles, in one
+  launch with the norm/RoPE/append epilogue or as partials and a finish launch:
+  the same contract (bit-exact on exact inputs, within one ulp plus the
   accumulation term on random ones) at 70-300 tokens and at 1024 tokens of
   hidden 5120 (two config-4 sequences), and the path taken is reported.
 """
@@ -150,8 +150,8 @@ def test_project_random_then_decode(device):
 @pytest.mark.parametrize("hidden,n_new", [(512, [1]), (1024, [30, 25, 15]), (1024, [20, 20]),
                                           (2048, [64, 1, 7]), (5120, [3, 70])])
 def test_project_chunks_and_splits(device, hidden, n_new):
-    """Steps of more than 64 tokens run in several launch pairs; hidden 512,
-    1024 and 2048 select 1, 2 and 4 splits."""
+    """Steps on both sides of 64 tokens: head tiles of one launch (hidden 512)
+    and products split in two or more for a finish launch."""
     rng = np.random.default_rng(33 + hidden)
     lengths = [int(x) for x in rng.integers(0, 300, len(n_new))]
     say(f"project_append hidden {hidden}, n_new {n_new}")
