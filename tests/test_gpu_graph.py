@@ -66,6 +66,42 @@ def test_graph_replay_many_pieces(device, lengths, split):
     _replay(device, lengths, split, False, steps=4, same_outputs=True, other_shape=False)
 
 
+@pytest.mark.parametrize("lengths,split", [([760], 16), ([600, 5, 77], 16), ([900, 5, 700, 30, 40, 77], 16),
+                                           ([1500, 900, 250, 256, 7, 20, 33, 64, 90, 15, 16, 17, 300, 1030], 16),
+                                           ([300, 1000], 0)])
+def test_graph_replay_gate(device, lengths, split):
+    """A gated decode recorded and replayed gives the eager call's bits, though
+    the two merge their pieces in different kernels."""
+    say(f"graph replay gate lengths={lengths} split={split}")
+    rng = np.random.default_rng(sum(lengths))
+    ids, o = [], 0
+    for L in lengths:
+        ids.append(list(range(o, o + L // 16 + 1)))
+        o += len(ids[-1])
+    cache, _, _ = build_cache(lengths, ids, extra_rows=1, rng=rng)
+    cache.set_decode_split(split)
+    B, stream = len(lengths), Stream()
+    for b, L in enumerate(lengths):
+        cache.set_len(b, L - 1)
+    cache.begin_step(list(range(B)), [1] * B, stream=stream.handle)
+    q, gate = [device.array(rng.standard_normal((B, H, D), dtype=np.float32).astype(np.float16)) for _ in range(2)]
+    eager, out = device.empty((B, H, D), np.float16), device.empty((B, H, D), np.float16)
+    cache.decode(0, q, eager, stream=stream.handle, gate=gate)
+    graph = cache.record_step(stream.handle)
+    cache.decode(0, q, out, stream=stream.handle, gate=gate)
+    graph.end()
+    for _ in range(2):
+        stream.synchronize()
+        out.copy_from(np.zeros((B, H, D), np.float16))
+        graph.launch()
+        stream.synchronize()
+        assert np.array_equal(out.numpy().view(np.uint16), eager.numpy().view(np.uint16))
+    graph.destroy()
+    stream.synchronize()
+    stream.destroy()
+    cache.destroy()
+
+
 @pytest.mark.parametrize("fused", [False, True])
 def test_graph_whole_form_past_64_pages(device, fused):
     """A step recorded in the whole-sequence form (longest sequence 1021
