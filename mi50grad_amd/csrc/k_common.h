@@ -263,7 +263,9 @@ __device__ __forceinline__ float sigmoid(float g) {
 // applied to the attention output, engine.py:2055-2056 after decode and
 // :3120-3121 after prefill), so the fused result is within one fp16 ulp of the
 // reference's two launches.  Infinite gates give the output and 0, NaN gives
-// NaN (the clamps propagate it).  With expf and the division, some 40
+// NaN (the clamps propagate it).  An infinite output gives NaN under gates
+// below -88.7, as infinity times a float32 0 does, and already from -87.4 on,
+// where the division left a subnormal.  With expf and the division, some 40
 // instructions per value, the gate was 43 of the 174 us of a prefill of 4 x
 // 512 tokens.
 __device__ __forceinline__ uint2 gate4(uint2 o, uint2 gw) {
