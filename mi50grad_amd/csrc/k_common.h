@@ -267,7 +267,10 @@ __device__ __forceinline__ float sigmoid(float g) {
 // below -88.7, as infinity times a float32 0 does, and already from -87.4 on,
 // where the division left a subnormal.  With expf and the division, some 40
 // instructions per value, the gate was 43 of the 174 us of a prefill of 4 x
-// 512 tokens.
+// 512 tokens.  A wave ends a unit with 64 values a lane one after another, so
+// each instruction counts: a layer over 181 tokens takes 101.9 us without the
+// correction, 102.6 with it and 104.9 with exp by n and f joined by ldexp (a
+// gated prefill of 100 tokens 28.0 and 29.7 without and with).
 __device__ __forceinline__ uint2 gate4(uint2 o, uint2 gw) {
     const half2_t hi = {static_cast<_Float16>(kGateClamp), static_cast<_Float16>(kGateClamp)};
     const uint32_t w[2] = {gw.x, gw.y}, ow[2] = {o.x, o.y};
